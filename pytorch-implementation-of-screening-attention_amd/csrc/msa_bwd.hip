@@ -12,12 +12,11 @@
 //   dr     = -sum 2 a (1-s) m dP,  dw = sum a^2 dP dm/dw
 //   dx     = (dx^ - x^ (x^.dx^)) / |x|   (|x| > eps),  dx^/eps otherwise
 // Only the 32x32 units the forward marked live in its bitmap are revisited;
-// each wave turns its bitmap row/column into a 64-bit ballot mask and walks
-// the set bits.  MFMA operands are the raw q, k, v values (exact in bf16),
-// loaded straight from global memory into operand registers, and the 1/|x|
+// each wave walks its bitmap row/column.  MFMA operands are the raw q, k, v
+// values (exact in bf16), staged in LDS a unit at a time and read in row and in
+// column order, and the 1/|x|
 // factors are applied in fp32 to the products, so no normalised copy is
-// rounded; dh is formed on the fly from y, dy and |h|.  Operands needed
-// transposed come from identity MFMAs on the same registers, per-row scale
+// rounded; dh is formed on the fly from y, dy and |h|.  Per-row scale
 // factors reach register order through a small LDS vector.  Key padding
 // (attention.py:185-188) enters as a zero 1/|k|, which gives s = 0 and so
 // alpha = 0 for those keys.
@@ -122,6 +121,17 @@ struct KeyRows {
   }
 };
 
+// D = 16 (DP = 32): rows of the product past D come from the repeated columns
+// of the staged rows; they are dropped here.
+template <typename T, int DP>
+__device__ inline void zero_past_d(f32x16 (&acc)[DP / 32], int D) {
+  if constexpr (DP == 32) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (Mma<T>::KS * creg_ks<T>(0, r) >= D) acc[0][r] = 0.0f;
+  }
+}
+
 // Writes dx = normalise-backward(dx^, x) (attention.py:156-158 under
 // autograd) for one row: dx^ in C-layout registers acc[dblk] whose rows are
 // tcol-ordered columns, x as the lane's raw operand fragments of the same row
@@ -132,10 +142,7 @@ __device__ inline void write_norm_bwd(const f32x16 (&acc)[DP / 32], const typena
                                       bool valid, int D, float eps, int half, T* out) {
   using M = Mma<T>;
   constexpr int NDH = DP / 32, NKS = DP / M::KS;
-  float ss = 0.0f;
-#pragma unroll
-  for (int ks = 0; ks < NKS; ++ks) ss = frag_dot(x[ks], x[ks], ss);
-  ss = half_sum(ss);
+  const float ss = half_sum(row_dot<T>(x, x));
   const float nx = sqrtf(ss);
   const float ix = 1.0f / fmaxf(nx, eps);
   float dot = 0.0f;
@@ -152,35 +159,48 @@ __device__ inline void write_norm_bwd(const f32x16 (&acc)[DP / 32], const typena
   });
 }
 
-// Waves per SIMD the backward kernels are register-budgeted for: two (256
-// registers a lane: the unit's operands, both accumulators and the scaled
-// products all stay in registers) where the bf16 working set allows, else one.
-template <typename T, int DP>
-constexpr int bwd_waves() { return sizeof(T) == 2 && DP <= 64 ? 2 : 1; }
-
 // ---------------------------------------------------------------------------
 // dQ (runs first).  One wave (a 64-thread block) per query unit: 32
 // consecutive queries of head (b,h), lane -> query i = 32*qu + l%32,
-// registers -> keys.  The wave walks its row of the live-unit bitmap; per
-// live key unit it loads the 32 raw K and V rows straight into MFMA operand
-// registers (A operands, row perm_row(l%32)), forms S^T = K Q^T and
-// dP^T = V dH^T, scales them by 1/|k|, 1/|v| (exchanged in register order
-// through a 32-float LDS vector), and accumulates dq^T += K^T (ds/|k|)^T with
-// K^T from an identity MFMA on the same registers.  Side output for
-// dkdv_kernel: dh (rounded to T, as the operand it becomes) and 1/|q| of the
-// unit's rows, written by every unit with a live key unit (the only rows
-// dkdv_kernel reads).
+// registers -> keys.  The wave walks its row of the live-unit bitmap; each
+// live key unit's raw K and V rows are staged in the wave's LDS (UnitTile),
+// the next unit's copies in flight behind the current one.  It forms S^T = K
+// Q^T and dP^T = V dH^T, scales them by 1/|k|, 1/|v| (exchanged in register
+// order through a 32-float LDS vector), and accumulates dq^T += K^T (ds/|k|)^T
+// with K^T read transposed from the staged rows.  Side output for dkdv_kernel:
+// dh (rounded to T, as the operand it becomes) and 1/|q| of the unit's rows,
+// written by every unit with a live key unit (the only rows dkdv_kernel
+// reads).  S > 1: as in the live pass, S waves share the row's live units and
+// wave 0 adds their partial dq, dr and dw in wave order.
 // ---------------------------------------------------------------------------
 template <typename T, int DP>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && DP <= 64 ? 3 : 1))) void dq_kernel(BwdKArgs a) {
+constexpr int dq_waves() { return sizeof(T) * DP <= 64 ? 3 : (sizeof(T) * DP <= 128 ? 2 : 1); }
+
+template <typename T, int DP, int S>
+__global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(dq_waves<T, DP>())))
+void dq_kernel(BwdKArgs a) {
   using M = Mma<T>;
   using frag = typename M::frag;
+  using U = UnitTile<T, DP>;
   constexpr int KS = M::KS, PER = M::PER, NKS = DP / KS, NDH = DP / 32, NC = 32 / KS;
-  __shared__ __attribute__((aligned(16))) float sk[32];  // 1/|k| (0 if padded or masked) of the unit's key rows
-  __shared__ __attribute__((aligned(16))) float sv[32];  // 1/|v|
-  __shared__ float mtab[128];  // soft-mask table of the current unit, then its dm/dw table (unit_mask_table)
-  __shared__ typename Mma<T>::frag qh[2 * (DP / Mma<T>::KS)][kWave];  // own raw q, dh operand fragments
-  const int lane = threadIdx.x, half = lane >> 5, l32 = lane & 31;
+  // per wave:
+  __shared__ __attribute__((aligned(16))) float sk_w[S][32];  // 1/|k| (0 if padded or masked) of the unit's key rows
+  __shared__ __attribute__((aligned(16))) float sv_w[S][32];  // 1/|v|
+  __shared__ float mtab_w[S][128];  // soft-mask table of the current unit, then its dm/dw table (unit_mask_table)
+  __shared__ __attribute__((aligned(16))) float sw_w[kPow2Rows<T> ? S : 1][32];   // fp16: the w of 1/|k| (Pow2Split)
+  __shared__ __attribute__((aligned(16))) f16 sc_w[kPow2Rows<T> ? S : 1][2][32];  // fp16: its powers of two
+  __shared__ __attribute__((aligned(1024))) char stage[S][2 * U::BYTES];  // the unit's K and V rows; then the partial dq
+  static_assert(NDH * 16 * kWave * 4 <= 2 * U::BYTES, "the partial dq fits the staged rows");
+  __shared__ frag hsh[NKS][kWave];  // own dh operand fragments (each wave writes the same ones)
+  const int lane = (int)(threadIdx.x & 63), half = lane >> 5, l32 = lane & 31;
+  const int wave = S > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+  float* sk = sk_w[wave];
+  float* sv = sv_w[wave];
+  float* mtab = mtab_w[wave];
+  char* kt = stage[wave];
+  char* vt = kt + U::BYTES;
+  LdsChar* const kt_at = (LdsChar*)&stage[0][0] + wave * 2 * U::BYTES;
+  LdsChar* const vt_at = kt_at + U::BYTES;
   int qu, bh;
   float head_r, head_w;
   xcd_interleave_ranked(a.r, a.w, a.H, qu, bh, head_r, head_w);
@@ -189,8 +209,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
   const HeadParams hp = head_params_rw(head_r, head_w, causal);
   const int i = qu * kUnit + l32;
   const bool valid = i < a.Tq;
-  const int ii = valid ? i : 0;
-  T* dqrow = (T*)a.dq + (((int64_t)b * a.Tq + ii) * a.H + h) * a.D;
+  auto dqrow = [&]() { return (T*)a.dq + (((int64_t)b * a.Tq + (valid ? i : 0)) * a.H + h) * a.D; };
 
   int ku_lo, ku_hi;
   {
@@ -207,14 +226,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
   int cur = walk.next();
   const int64_t nbh = (int64_t)a.B * a.H;
   const int nqu = 2 * a.nqt;
-  if (cur < 0) {  // wave-uniform: no live key unit, dq = 0 and no share of dr, dw
+  if (cur < 0) {  // block-uniform: no live key unit, dq = 0 and no share of dr, dw
+    if (wave != 0) return;
     if (valid)
 #pragma unroll
       for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int d = 32 * dblk + 8 * g + 4 * half;
-          if (d < a.D) store4(dqrow + d, 0.0f, 0.0f, 0.0f, 0.0f);
+          if (d < a.D) store4(dqrow() + d, 0.0f, 0.0f, 0.0f, 0.0f);
         }
     if (lane == 0) {
       a.part[(int64_t)bh * nqu + qu] = 0.0f;
@@ -222,24 +242,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
     }
     return;
   }
+  for (int w = 0; w < wave && cur >= 0; ++w) cur = walk.next();  // S > 1: the wave's first unit
 
-  // key row of this lane in unit u: 32u + perm_row(l32), read as row Tk-1
-  // past Tk (its 1/|k| is then 0, so it contributes nothing); the lane's
-  // chunks from a wave-uniform row base plus a 32-bit lane offset
+  // key row of this lane in unit u: 32u + perm_row(l32)
   const int m = perm_row(l32);
-  const T* kb0 = (const T*)a.k + b * a.ks.sb + h * a.ks.sh;
-  const T* vb0 = (const T*)a.v + b * a.vs.sb + h * a.vs.sh;
-  auto load_rows = [&](const T* base, int64_t st, int u, frag (&f)[NKS]) {
-    const int r = u * kUnit + m < a.Tk ? m : a.Tk - 1 - u * kUnit;
-    const uint32_t off = (uint32_t)(((int64_t)r * st + PER * half) * (int64_t)sizeof(T));
-    const char* p = (const char*)(base + (int64_t)u * kUnit * st) + off;
-    // chunks past D (D = 16 < DP = 32 only) re-read chunk 0; zero_tail clears them
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const int c = DP == 32 && KS * ks >= a.D ? 0 : KS * ks;
-      f[ks] = M::load((const T*)(p + c * (int)sizeof(T)));
-    }
-  };
+  const typename U::Source ksrc((const T*)a.k + b * a.ks.sb + h * a.ks.sh, a.ks.st, a.Tk, a.D, lane);
+  const typename U::Source vsrc((const T*)a.v + b * a.vs.sb + h * a.vs.sh, a.vs.st, a.Tk, a.D, lane);
+  const uint32_t rb = U::row_base(lane), cb = U::col_base(lane);
+  // D = 16: the staged columns past D repeat the first ones
   auto zero_tail = [&](frag (&f)[NKS]) {
     if constexpr (DP == 32) {
 #pragma unroll
@@ -248,35 +258,36 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
     }
   };
   // 1/|k| is 0 for keys past Tk and for masked keys
-  auto key_ok = [&](int u) {
+  auto key_mask = [&](int u) -> unsigned {  // the mask byte, tested when the unit is computed
     const int j = u * kUnit + m;
-    return j < a.Tk && !(a.kpm != nullptr && a.kpm[(int64_t)b * a.Tk + j] != 0);
+    return a.kpm != nullptr && j < a.Tk ? a.kpm[(int64_t)b * a.Tk + j] : 0u;
   };
 
-  // own queries' rows first, then the first key unit's rows behind them;
-  // the raw q and dh operand fragments are kept in LDS (read back per key
-  // unit), which leaves registers for three waves per SIMD
-  frag kc[NKS], vc[NKS];
+  // own queries' rows first, then the first key unit's copies behind them
+  frag qf[NKS];  // raw q operand fragments; those of dh are kept in LDS (read back per unit)
   float iql;
-  bool kok;
+  unsigned kmask = 0u;
   {
     QueryRows<T, DP> qr;
     qr.load(a, b, h, bh, i, half);
-    load_rows(kb0, a.ks.st, cur, kc);
-    load_rows(vb0, a.vs.st, cur, vc);
-    kok = key_ok(cur);
+    if (cur >= 0) {
+      ksrc.issue(kt_at, cur);
+      vsrc.issue(vt_at, cur);
+      kmask = key_mask(cur);
+    }
     iql = qr.finish(a.eps);
     // dh and 1/|q| of this unit's rows for dkdv_kernel (zero past Tq)
     T* dst = (T*)a.dh + ((int64_t)bh * a.Tq_pad + i) * DP;
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
-      qh[ks][lane] = qr.q.f[ks];
-      qh[NKS + ks][lane] = qr.dh.f[ks];
-      *reinterpret_cast<frag*>(dst + KS * ks + PER * half) = qr.dh.f[ks];
+      qf[ks] = qr.q.f[ks];
+      hsh[ks][lane] = qr.dh.f[ks];
+      if (wave == 0) *reinterpret_cast<frag*>(dst + KS * ks + PER * half) = qr.dh.f[ks];
     }
-    if (half == 0) a.iqs[(int64_t)bh * a.Tq_pad + i] = valid ? iql : 0.0f;
+    if (wave == 0 && half == 0) a.iqs[(int64_t)bh * a.Tq_pad + i] = valid ? iql : 0.0f;
   }
   const float thq = hp.thr / iql;  // s > thr  <=>  (q . k)/|k| > thr |q|
+  const float riq = hp.r * iql;
   float dr_acc = 0.0f, dw_acc = 0.0f;  // this unit's share of dr, dw
   f32x16 adq[NDH];
 #pragma unroll
@@ -284,58 +295,84 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
 #pragma unroll
     for (int r = 0; r < 16; ++r) adq[dblk][r] = 0.0f;
 
-  for (;;) {
+  while (cur >= 0) {
     const int k0 = cur * kUnit;
     // the unit's mask tables first, while few values are live (the LDS sync
     // after the products below covers these writes too; this iteration's
     // writes follow the previous one's reads in the wave's LDS order)
     unit_mask_table<true>(mtab, mtab + 64, qu * kUnit - k0 - 31, hp, lane);
-    const int nxt = walk.next();
-    zero_tail(kc);
-    zero_tail(vc);
+    wait_vmcnt<0>();  // the unit's rows have landed
     // register r -> key k0 + rowof(r, half), lane -> query i
-    f32x16 s, dp;
-    float s2k = 0.0f, s2v = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { s[r] = 0.0f; dp[r] = 0.0f; }
+    f32x16 s, slo, dp;  // fp32: s + slo
+    float ikl, iv;  // 1/|k|, 1/|v| of this lane's key row m
+    frag ka[NDH * NC];
     {
-      frag g[NKS];
+      float s2k, s2v;
+      {
+        frag kf[NKS];
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) g[ks] = qh[ks][lane];
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        s = M::mma_ng(kc[ks], g[ks], s);
-        s2k = frag_dot(kc[ks], kc[ks], s2k);
+        for (int ks = 0; ks < NKS; ++ks) kf[ks] = U::row_frag(kt, rb, ks);
+        zero_tail(kf);
+        s = unit_product<T>(kf, qf, &slo);
+        s2k = row_dot<T>(kf, kf);
+        guard_run(kf, s);
       }
-      guard_frags(g);
+      __builtin_amdgcn_sched_barrier(0);
+      {
+        frag vf[NKS], hf[NKS];
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) g[ks] = qh[NKS + ks][lane];
+        for (int ks = 0; ks < NKS; ++ks) vf[ks] = U::row_frag(vt, rb, ks);
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        dp = M::mma_ng(vc[ks], g[ks], dp);
-        s2v = frag_dot(vc[ks], vc[ks], s2v);
+        for (int ks = 0; ks < NKS; ++ks) hf[ks] = hsh[ks][lane];
+        zero_tail(vf);
+        dp = unit_product<T>(vf, hf);
+        s2v = row_dot<T>(vf, vf);
+        guard_run(vf, dp);
+        guard_keep(hf);
       }
-      guard_frags(g);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) ka[dblk * NC + c] = U::col_frag(kt, cb, dblk, c);
+      ikl = k0 + m < a.Tk && kmask == 0u ? inv_len_of<T>(half_sum(s2k), a.eps) : 0.0f;
+      iv = inv_len_of<T>(half_sum(s2v), a.eps);
     }
-    guard_frags(vc);
-    s2k = half_sum(s2k);
-    s2v = half_sum(s2v);
-    const float ikl = kok ? inv_len(s2k, a.eps) : 0.0f;  // this lane's key row m
-    {
-      const float iv = inv_len(s2v, a.eps);
-      wave_lds_sync();
-      if (half == 0) { sk[m] = ikl; sv[m] = iv; }
-      wave_lds_sync();
+    // every read of the staged rows has returned: the next unit's copies run
+    // behind the rest of this unit's work
+    int nxt = -1;  // this wave's next unit: S positions on in the row's walk
+    for (int w = 0; w < S; ++w) {
+      nxt = walk.next();
+      if (nxt < 0) break;
     }
+    wave_lds_sync();
+    if (nxt >= 0) {
+      ksrc.issue(kt_at, nxt);
+      vsrc.issue(vt_at, nxt);
+      kmask = key_mask(nxt);
+    }
+    if (half == 0) {
+      sk[m] = ikl;
+      sv[m] = iv;
+      if constexpr (kPow2Rows<T>) {
+        const Pow2Split p(ikl);
+        sw_w[wave][m] = p.w;
+        sc_w[wave][0][m] = (f16)p.c1;
+        sc_w[wave][1][m] = (f16)p.c2;
+      }
+    }
+    wave_lds_sync();
     // scaled in place: s = (q . k)/|k|, dp = dH . v^
     {
       float sc[16];
       read_row_scales(sk, half, sc);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] *= sc[r];
+      for (int r = 0; r < 16; ++r) scale_pair<T>(s, slo, r, sc[r]);
+      __builtin_amdgcn_sched_barrier(0);
       read_row_scales(sv, half, sc);
 #pragma unroll
       for (int r = 0; r < 16; ++r) dp[r] *= sc[r];
+      __builtin_amdgcn_sched_barrier(0);
     }
     // every lane forms its pair's terms branch-free (a = 0 below the
     // threshold, the mask and dm/dw, 0 outside the window, from the unit's
@@ -347,16 +384,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
       // entry 23 - (16(r/8) + r%8) of each table: constant offsets from one base
       const float* mrow = mtab + (l32 - 8 * half + 8);
       // (rows past Tq hold q = 0, so s = 0 and a = 1 - r <= 0: no term)
+      // with um = a m dP: ds = 2r um (2r enters once, in the epilogue), dr
+      // = -2 um (1 - s) = -(2/r) um (1 - a), dw = a^2 dP dm/dw
       auto body = [&](int r) {
         const int off = 16 * (r >> 3) + (r & 7);
-        const float sv = s[r] * iql;
-        const float av = fmaxf(trim(sv, hp.r), 0.0f);
-        float g = dp[r];
-        if (a.drop.on) g *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
-        const float t = 2.0f * av * mrow[23 - off] * g;
-        dr_acc -= t * (1.0f - sv);
-        dw_acc += av * av * g * mrow[64 + 23 - off];
-        dp[r] = hp.r * t;
+        const float av = pair_root<T>(s[r], slo[r], iql, riq, hp.r);
+        float u = av * dp[r];
+        if (a.drop.on) u *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
+        const float um = u * mrow[23 - off];
+        dr_acc = fmaf(um, 1.0f - av, dr_acc);
+        dw_acc = fmaf(u * av, mrow[64 + 23 - off], dw_acc);
+        dp[r] = um;
       };
       if (a.drop.on) {  // the pair's hash only where some lane may pass
         const uint32_t pm0 = pass_mask(s, thq);
@@ -366,56 +404,70 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
           if (((pm0 >> r) & 1u) == 0u) dp[r] = 0.0f;
       } else {  // every register: a = 0 gives no term, and no mask or branches
 #pragma unroll
-        for (int r = 0; r < 16; ++r) body(r);
+        for (int r = 0; r < 16; ++r) {
+          body(r);
+          if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four registers' terms live at a time
+        }
       }
     }
-    // dq^T[d][i] += sum_j K^T[d][j] (ds/|k|)^T[j][i], K^T by identity from
-    // the key rows, one 32-column block of d at a time (fp16: K^T takes
-    // 1/|k| instead, below)
-    if constexpr (!kScaleRowsNotWeights<T>) {
+    // dq^T[d][i] += sum_j K^T[d][j] (ds/|k|)^T[j][i] (fp16: 1/|k|'s power of
+    // two goes to the K columns, the rest to ds)
+    {
       float ksc[16];
-      read_row_scales(sk, half, ksc);
+      if constexpr (kPow2Rows<T>) read_row_scales(sw_w[wave], half, ksc);
+      else read_row_scales(sk, half, ksc);
 #pragma unroll
       for (int r = 0; r < 16; ++r) dp[r] *= ksc[r];
+    }
+    if constexpr (kPow2Rows<T>) {
+      const bool tiny = __ballot(ikl > 32768.0f) != 0ull;  // rows shorter than 2^-15
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int dblk = 0; dblk < NDH; ++dblk) {
+          scale_slots(ka[dblk * NC + c], sc_w[wave][0], c, half);
+          if (tiny) scale_slots(ka[dblk * NC + c], sc_w[wave][1], c, half);
+        }
     }
     frag db[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) db[c] = M::pack(dp, c * PER);
-    frag id[NC];  // identity slices, held (and guarded) as named operands
 #pragma unroll
-    for (int c = 0; c < NC; ++c) id[c] = ident_frag<T>(c, lane);
+    for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int dblk = 0; dblk < NDH; ++dblk) {
-      frag kt[NC];
-      f32x16 tr;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) tr[r] = 0.0f;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) tr = M::mma_ng(kc[dblk * NC + c], id[c], tr);
-      if constexpr (kScaleRowsNotWeights<T>) scale_rows_fp32(tr, sk, half);
-#pragma unroll
-      for (int c = 0; c < NC; ++c) kt[c] = M::pack(tr, c * PER);
-#pragma unroll
-      for (int c = 0; c < NC; ++c) adq[dblk] = M::mma_ng(kt[c], db[c], adq[dblk]);
-      guard_frags(kt);
-    }
-    guard_frags(kc);
-    guard_frags(db);
-    guard_frags(id);
-    if (nxt < 0) break;
+      for (int dblk = 0; dblk < NDH; ++dblk) adq[dblk] = M::mma_ng(ka[dblk * NC + c], db[c], adq[dblk]);
+    guard_run(ka, adq[NDH - 1]);
+    guard_keep(db);
     cur = nxt;
-    load_rows(kb0, a.ks.st, cur, kc);
-    load_rows(vb0, a.vs.st, cur, vc);
-    kok = key_ok(cur);
   }
-  {
-    frag x[NKS];
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) x[ks] = qh[ks][lane];
-    write_norm_bwd<T, DP>(adq, x, valid, a.D, a.eps, half, dqrow);
-  }
-  dr_acc = wave_sum(dr_acc);
+  dr_acc = wave_sum(dr_acc) * (-2.0f / hp.r);
   dw_acc = wave_sum(dw_acc);
+  if constexpr (S > 1) {
+    auto part = [&](int w) { return reinterpret_cast<float(*)[kWave]>(stage[w]); };
+    if (wave > 0) {
+#pragma unroll
+      for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part(wave)[dblk * 16 + r][lane] = adq[dblk][r];
+      if (lane == 0) { sk[0] = dr_acc; sv[0] = dw_acc; }
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    for (int w = 1; w < S; ++w) {
+#pragma unroll
+      for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) adq[dblk][r] += part(w)[dblk * 16 + r][lane];
+      dr_acc += sk_w[w][0];
+      dw_acc += sv_w[w][0];
+    }
+  }
+#pragma unroll
+  for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) adq[dblk][r] *= 2.0f * hp.r;
+  zero_past_d<T, DP>(adq, a.D);
+  write_norm_bwd<T, DP>(adq, qf, valid, a.D, a.eps, half, dqrow());
   if (lane == 0) {
     a.part[(int64_t)bh * nqu + qu] = dr_acc;
     a.part[nbh * nqu + (int64_t)bh * nqu + qu] = dw_acc;
@@ -426,23 +478,44 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
 // dK, dV (runs after dq_kernel).  One wave (a 64-thread block) per key unit:
 // 32 consecutive keys of head (b,h), lane -> key j = 32*ku + l%32 of the C
 // blocks, registers -> queries.  The wave walks its column of the live-unit
-// bitmap; per live query unit it loads the raw Q rows and the dh rows and
-// 1/|q| that dq_kernel left in the workspace straight into MFMA operand
-// registers (A operands, row perm_row(l%32)), forms S = Q K^T and dP = dH V^T
-// with its own raw K, V rows as B operands, and accumulates
-// dv^T += dH^T P and dk^T += Q^T (ds/|q|) with dH^T, Q^T from identity MFMAs
-// on the same registers.  1/|q| reaches register order through a 32-float
-// LDS vector.  The wave finishes dk, dv and its (dr, dw) partial.
+// bitmap; each live query unit's raw Q rows and the dh rows that dq_kernel
+// left in the workspace are staged in the wave's LDS (UnitTile), the next
+// unit's copies in flight behind the current one.  It forms S = Q K^T and dP =
+// dH V^T with its own raw K, V rows as B operands, and accumulates dv^T +=
+// dH^T P and dk^T += Q^T (ds/|q|) with dH^T, Q^T read transposed from the
+// staged rows.  1/|q| reaches register order through a 32-float LDS vector.
+// S > 1: S waves share the column's live units; wave 0 adds their partial dk,
+// dv in wave order.
 // ---------------------------------------------------------------------------
+// Waves per SIMD: two where both accumulators, the unit's fragments and their
+// transposes fit 256 registers a lane.
 template <typename T, int DP>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(bwd_waves<T, DP>()))) void dkdv_kernel(BwdKArgs a) {
+constexpr int dkdv_waves() { return sizeof(T) * DP <= 128 ? 2 : 1; }
+template <typename T>
+constexpr bool kLateColumns = sizeof(T) == 4;
+
+template <typename T, int DP, int S>
+__global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(dkdv_waves<T, DP>())))
+void dkdv_kernel(BwdKArgs a) {
   using M = Mma<T>;
   using frag = typename M::frag;
+  using U = UnitTile<T, DP>;
   constexpr int KS = M::KS, PER = M::PER, NKS = DP / KS, NDH = DP / 32, NC = 32 / KS;
-  __shared__ __attribute__((aligned(16))) float sq[32];  // 1/|q| of the current query unit's rows
-  __shared__ float mt[64];  // soft-mask table of the current unit (unit_mask_table)
-  __shared__ typename Mma<T>::frag kvs[2 * (DP / Mma<T>::KS)][kWave];  // own raw k, v operand fragments
-  const int lane = threadIdx.x, half = lane >> 5, l32 = lane & 31;
+  // per wave:
+  __shared__ __attribute__((aligned(16))) float sq_w[S][32];  // 1/|q| of the current query unit's rows
+  __shared__ float mt_w[S][64];  // soft-mask table of the current unit (unit_mask_table)
+  __shared__ __attribute__((aligned(16))) float sw_w[kPow2Rows<T> ? S : 1][32];   // fp16: the w of 1/|q| (Pow2Split)
+  __shared__ __attribute__((aligned(16))) f16 sc_w[kPow2Rows<T> ? S : 1][2][32];  // fp16: its powers of two
+  __shared__ __attribute__((aligned(1024))) char stage[S][2 * U::BYTES];  // the unit's Q and dh rows; then partial dk, dv
+  static_assert(NDH * 16 * kWave * 4 <= 2 * U::BYTES, "a partial dk fits the staged rows");
+  const int lane = (int)(threadIdx.x & 63), half = lane >> 5, l32 = lane & 31;
+  const int wave = S > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+  float* sq = sq_w[wave];
+  float* mt = mt_w[wave];
+  char* qt = stage[wave];
+  char* ht = qt + U::BYTES;
+  LdsChar* const qt_at = (LdsChar*)&stage[0][0] + wave * 2 * U::BYTES;
+  LdsChar* const ht_at = qt_at + U::BYTES;
   int ku, bh;
   float head_r, head_w;
   xcd_interleave_ranked(a.r, a.w, a.H, ku, bh, head_r, head_w);
@@ -457,7 +530,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(bwd_waves<T,
   const bool jvalid = j < a.Tk;
   const int jj = jvalid ? j : 0;
   const int64_t orow = (((int64_t)b * a.Tk + jj) * a.H + h) * a.D;
-  if (ku == 2 * a.nkt - 1 && bh < a.H) {
+  if (ku == 2 * a.nkt - 1 && bh < a.H && wave == 0) {
     // one wave per head: dr, dw from dq_kernel's per-query-unit shares
     // (complete: dq_kernel ran first), summed in a fixed order
     const int64_t nbh = (int64_t)a.B * a.H;
@@ -490,8 +563,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(bwd_waves<T,
   const uint32_t* bcol = a.bits + (int64_t)bh * 2 * a.nqt * a.nku_words + (ku >> 5);
   ColWalk walk(bcol, a.nku_words, ku & 31, qu_lo, qu_hi);
   int cur = walk.next();
-  if (cur < 0) {  // wave-uniform: no live query unit, dk = dv = 0
-    if (jvalid)
+  if (cur < 0) {  // block-uniform: no live query unit, dk = dv = 0
+    if (jvalid && wave == 0)
 #pragma unroll
       for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
@@ -504,28 +577,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(bwd_waves<T,
         }
     return;
   }
+  for (int w = 0; w < wave && cur >= 0; ++w) cur = walk.next();  // S > 1: the wave's first unit
 
-  // query row of this lane in unit u: 32u + perm_row(l32).  Raw q rows past
-  // Tq read row Tq-1; their 1/|q| and dh rows (workspace, zero past Tq) are
-  // 0, so they contribute nothing.  A wave-uniform row base plus a 32-bit
-  // lane offset per operand.
-  const int m = perm_row(l32);
-  const T* qb0 = (const T*)a.q + b * a.qs.sb + h * a.qs.sh;
-  const T* hb0 = (const T*)a.dh + (int64_t)bh * a.Tq_pad * DP;
+  // Raw q rows past Tq read row Tq-1; their 1/|q| and dh rows (workspace,
+  // zero past Tq) are 0, so they contribute nothing.
+  const typename U::Source qsrc((const T*)a.q + b * a.qs.sb + h * a.qs.sh, a.qs.st, a.Tq, a.D, lane);
+  const typename U::Source hsrc((const T*)a.dh + (int64_t)bh * a.Tq_pad * DP, DP, (int)a.Tq_pad, DP, lane);
   const float* iq0 = a.iqs + (int64_t)bh * a.Tq_pad;
-  auto load_unit = [&](int u, frag (&qf)[NKS], frag (&hf)[NKS], float& iqv) {
-    const int r = u * kUnit + m < a.Tq ? m : a.Tq - 1 - u * kUnit;
-    const uint32_t qoff = (uint32_t)(((int64_t)r * a.qs.st + PER * half) * (int64_t)sizeof(T));
-    const char* pq = (const char*)(qb0 + (int64_t)u * kUnit * a.qs.st) + qoff;
-    const char* ph = (const char*)(hb0 + (int64_t)u * kUnit * DP) + (uint32_t)((m * DP + PER * half) * (int)sizeof(T));
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const int c = DP == 32 && KS * ks >= a.D ? 0 : KS * ks;  // chunks past D re-read chunk 0 (cleared at use)
-      qf[ks] = M::load((const T*)(pq + c * (int)sizeof(T)));
-      hf[ks] = M::load((const T*)(ph + KS * ks * (int)sizeof(T)));
-    }
-    iqv = iq0[(int64_t)u * kUnit + l32];  // lanes l and l+32 read the same row
-  };
+  const uint32_t rb = U::row_base(lane), cb = U::col_base(lane);
+  // D = 16: the staged columns past D repeat the first ones (dh rows hold DP)
   auto zero_tail = [&](frag (&f)[NKS]) {
     if constexpr (DP == 32) {
 #pragma unroll
@@ -534,70 +594,95 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(bwd_waves<T,
     }
   };
 
-  // own keys as raw B operands (lane -> key), kept in LDS (read back per
-  // query unit; the registers hold the next unit's rows instead), with 1/|k|
-  // (0 if padded or masked) and 1/|v|; their loads go first, the first query
-  // unit's behind
-  frag qf[NKS], hf[NKS];
-  float ikl, ivl, iqv;
-  {
-    KeyRows<T, DP> kr;
-    kr.load(a, b, h, j, half);
-    load_unit(cur, qf, hf, iqv);
-    kr.finish(a.eps, ikl, ivl);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      kvs[ks][lane] = kr.k.f[ks];
-      kvs[NKS + ks][lane] = kr.v.f[ks];
-    }
+  // own keys as raw B operands (lane -> key), with 1/|k| (0 if padded or
+  // masked) and 1/|v|; their loads go first, the first query unit's behind
+  KeyRows<T, DP> kr;
+  float ikl, ivl, iqv = 0.0f;
+  kr.load(a, b, h, j, half);
+  if (cur >= 0) {
+    qsrc.issue(qt_at, cur);
+    hsrc.issue(ht_at, cur);
+    iqv = iq0[(int64_t)cur * kUnit + l32];  // lanes l and l+32 read the same row
   }
+  kr.finish(a.eps, ikl, ivl);
   f32x16 acc_k[NDH], acc_v[NDH];
 #pragma unroll
   for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { acc_k[dblk][r] = 0.0f; acc_v[dblk][r] = 0.0f; }
+  const float rik = hp.r * ikl;
   const float thk = hp.thr / ikl;  // s > thr  <=>  (q . k)/|q| > thr |k|  (+inf for masked keys)
 
-  for (;;) {
+  while (cur >= 0) {
     const int q0 = cur * kUnit;
-    // the next unit's rows load while this one is computed (past the last
-    // unit, the current one again, a cache hit: every iteration then waits
-    // for the same count)
-    const int nxt = walk.next();
-    frag qn[NKS], hn[NKS];
-    float iqn;
-    load_unit(nxt >= 0 ? nxt : cur, qn, hn, iqn);
-    zero_tail(qf);
-    wave_lds_sync();
-    if (half == 0) sq[l32] = iqv;
-    unit_mask_table<false>(mt, nullptr, q0 - k0 - 31, hp, lane);
-    wave_lds_sync();
-    // register r -> query q0 + rowof(r, half), lane -> key j.  Scaled in
-    // place: s = (q . k)/|q|, dp = (dh . v)/|v|.
-    f32x16 s, dp;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { s[r] = 0.0f; dp[r] = 0.0f; }
-    {
-      frag g[NKS];
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) g[ks] = kvs[ks][lane];
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) s = M::mma_ng(qf[ks], g[ks], s);
-      guard_frags(g);
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) g[ks] = kvs[NKS + ks][lane];
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) dp = M::mma_ng(hf[ks], g[ks], dp);
-      guard_frags(g);
-    }
-    {
-      float sc[16];
-      read_row_scales(sq, half, sc);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        s[r] *= sc[r];
-        dp[r] *= ivl;
+    wait_vmcnt<0>();  // the unit's rows have landed
+    const float iqc = iqv;
+    if (half == 0) {
+      sq[l32] = iqc;
+      if constexpr (kPow2Rows<T>) {
+        const Pow2Split p(iqc);
+        sw_w[wave][l32] = p.w;
+        sc_w[wave][0][l32] = (f16)p.c1;
+        sc_w[wave][1][l32] = (f16)p.c2;
       }
+    }
+    unit_mask_table<false>(mt, nullptr, q0 - k0 - 31, hp, lane);
+    // register r -> query q0 + rowof(r, half), lane -> key j
+    f32x16 s, slo, dp;  // fp32: s + slo
+    {
+      frag f[NKS];
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) f[ks] = U::row_frag(qt, rb, ks);
+      zero_tail(f);
+      s = unit_product<T>(f, kr.k.f, &slo);
+      guard_run(f, s);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      frag f[NKS];
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks) f[ks] = U::row_frag(ht, rb, ks);
+      dp = unit_product<T>(f, kr.v.f);
+      guard_run(f, dp);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    int nxt = -1;  // this wave's next unit: S positions on in the column's walk
+    for (int w = 0; w < S; ++w) {
+      nxt = walk.next();
+      if (nxt < 0) break;
+    }
+    // once every read of the staged rows has returned, the next unit's copies
+    // run behind the rest of this unit's work (fp32 reads the columns only
+    // where it uses them: two transposed operands would not fit the registers)
+    frag qa[kLateColumns<T> ? 1 : NDH * NC], ha[kLateColumns<T> ? 1 : NDH * NC];
+    auto copy_next = [&]() {
+      wave_lds_sync();
+      if (nxt >= 0) {
+        qsrc.issue(qt_at, nxt);
+        hsrc.issue(ht_at, nxt);
+        iqv = iq0[(int64_t)nxt * kUnit + l32];
+      }
+    };
+    if constexpr (!kLateColumns<T>) {
+#pragma unroll
+      for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          ha[dblk * NC + c] = U::col_frag(ht, cb, dblk, c);
+          qa[dblk * NC + c] = U::col_frag(qt, cb, dblk, c);
+        }
+      copy_next();
+    } else {
+      wave_lds_sync();
+    }
+    // scaled in place: s = (q . k)/|q|; dp = dh . v takes its lane's 1/|v| and
+    // 2r once, in the epilogue (fp16: 1/|v| here, to keep ds in range)
+    float qsc[16];
+    read_row_scales(sq, half, qsc);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      scale_pair<T>(s, slo, r, qsc[r]);
+      if constexpr (kPow2Rows<T>) dp[r] *= ivl;
     }
     // every lane forms its pair's weight and ds branch-free (the mask, 0
     // outside the window, from the unit's table: entry 16(r/8) + r%8 + 8half
@@ -608,12 +693,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(bwd_waves<T,
       const float* mrow = mt + (8 * half - l32 + 31);
       auto body = [&](int r) {
         const int off = 16 * (r >> 3) + (r & 7);
-        const float av = fmaxf(trim(s[r] * ikl, hp.r), 0.0f);
+        const float av = pair_root<T>(s[r], slo[r], ikl, rik, hp.r);
         float mk = mrow[off];
         if (a.drop.on) mk *= dropout_factor(a.drop, bh, q0 + 8 * half + off, j);
         const float am = av * mk;
         s[r] = av * am;
-        dp[r] = 2.0f * hp.r * am * dp[r];
+        dp[r] = am * dp[r];
       };
       if (a.drop.on) {  // the pair's hash only where some lane may pass
         const uint32_t pm0 = pass_mask(s, thk);
@@ -626,70 +711,89 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(bwd_waves<T,
         for (int r = 0; r < 16; ++r) body(r);
       }
     }
-    // ds/|q| (fp16: Q^T takes 1/|q| instead, below)
-    if constexpr (!kScaleRowsNotWeights<T>) {
-      float qsc[16];
-      read_row_scales(sq, half, qsc);
+    // ds/|q| (fp16: 1/|q|'s power of two goes to the Q columns, the rest here)
+    if constexpr (kPow2Rows<T>) read_row_scales(sw_w[wave], half, qsc);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) dp[r] *= qsc[r];
+    for (int r = 0; r < 16; ++r) dp[r] *= qsc[r];
+    if constexpr (kPow2Rows<T>) {
+      const bool tiny = __ballot(iqc > 32768.0f) != 0ull;  // rows shorter than 2^-15
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int dblk = 0; dblk < NDH; ++dblk) {
+          scale_slots(qa[dblk * NC + c], sc_w[wave][0], c, half);
+          if (tiny) scale_slots(qa[dblk * NC + c], sc_w[wave][1], c, half);
+        }
     }
     // dv^T[d][j] += sum_i dH^T[d][i] P[i][j];  dk^T[d][j] += sum_i Q^T[d][i] (ds/|q|)[i][j]
-    // with dH^T, Q^T from identity products on the row registers, one
-    // 32-column block of d at a time
-    frag pb[NC], db[NC], id[NC];
+    frag pb[NC], db[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       pb[c] = M::pack(s, c * PER);
       db[c] = M::pack(dp, c * PER);
-      id[c] = ident_frag<T>(c, lane);  // held (and guarded) as named operands
     }
+    if constexpr (kLateColumns<T>) {
 #pragma unroll
-    for (int dblk = 0; dblk < NDH; ++dblk) {
+      for (int op = 0; op < 2; ++op) {
 #pragma unroll
-      for (int op = 0; op < 2; ++op) {  // 0: dH^T P -> dv, 1: Q^T dS -> dk
-        frag t[NC];
-        f32x16 tr;
+        for (int dblk = 0; dblk < NDH; ++dblk) {
+          frag f[NC];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) tr[r] = 0.0f;
+          for (int c = 0; c < NC; ++c) f[c] = U::col_frag(op == 0 ? ht : qt, cb, dblk, c);
+          f32x16& acc = op == 0 ? acc_v[dblk] : acc_k[dblk];
 #pragma unroll
-        for (int c = 0; c < NC; ++c)
-          tr = M::mma_ng(op == 0 ? hf[dblk * NC + c] : qf[dblk * NC + c], id[c], tr);
-        if constexpr (kScaleRowsNotWeights<T>)
-          if (op == 1) scale_rows_fp32(tr, sq, half);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) t[c] = M::pack(tr, c * PER);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          if (op == 0) acc_v[dblk] = M::mma_ng(t[c], pb[c], acc_v[dblk]);
-          else acc_k[dblk] = M::mma_ng(t[c], db[c], acc_k[dblk]);
+          for (int c = 0; c < NC; ++c) acc = M::mma_ng(f[c], op == 0 ? pb[c] : db[c], acc);
+          guard_run(f, acc);
         }
-        guard_frags(t);
       }
-    }
-    guard_frags(qf);
-    guard_frags(hf);
-    guard_frags(pb);
-    guard_frags(db);
-    guard_frags(id);
-    if (nxt < 0) break;
-    cur = nxt;
+      guard_keep(pb);
+      guard_keep(db);
+      copy_next();
+    } else {
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      qf[ks] = qn[ks];
-      hf[ks] = hn[ks];
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int dblk = 0; dblk < NDH; ++dblk) {
+          acc_v[dblk] = M::mma_ng(ha[dblk * NC + c], pb[c], acc_v[dblk]);
+          acc_k[dblk] = M::mma_ng(qa[dblk * NC + c], db[c], acc_k[dblk]);
+        }
+      guard_run(qa, acc_k[NDH - 1]);
+      guard_keep(ha);
+      guard_keep(pb);
+      guard_keep(db);
     }
-    iqv = iqn;
+    cur = nxt;
   }
 
-  {
-    frag x[NKS];
+  if constexpr (S > 1) {
+    auto part = [&](int w) { return reinterpret_cast<float(*)[kWave]>(stage[w]); };
+    auto add_up = [&](f32x16 (&acc)[NDH]) {
+      if (wave > 0)
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) x[ks] = kvs[ks][lane];
-    write_norm_bwd<T, DP>(acc_k, x, jvalid, a.D, a.eps, half, (T*)a.dk + orow);
+        for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) x[ks] = kvs[NKS + ks][lane];
-    write_norm_bwd<T, DP>(acc_v, x, jvalid, a.D, a.eps, half, (T*)a.dv + orow);
+          for (int r = 0; r < 16; ++r) part(wave)[dblk * 16 + r][lane] = acc[dblk][r];
+      __syncthreads();
+      if (wave == 0)
+        for (int w = 1; w < S; ++w)
+#pragma unroll
+          for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[dblk][r] += part(w)[dblk * 16 + r][lane];
+      __syncthreads();
+    };
+    add_up(acc_k);
+    add_up(acc_v);
+    if (wave > 0) return;
   }
+#pragma unroll
+  for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc_k[dblk][r] *= kPow2Rows<T> ? 2.0f * hp.r : 2.0f * hp.r * ivl;
+  zero_past_d<T, DP>(acc_k, a.D);
+  zero_past_d<T, DP>(acc_v, a.D);
+  write_norm_bwd<T, DP>(acc_k, kr.k.f, jvalid, a.D, a.eps, half, (T*)a.dk + orow);
+  write_norm_bwd<T, DP>(acc_v, kr.v.f, jvalid, a.D, a.eps, half, (T*)a.dv + orow);
 }
 
 // Workspace: [dr/dw partials][dh][1/|q|], each 256-byte aligned.
@@ -718,15 +822,27 @@ static hipError_t launch_bwd_t(const BwdCall& c) {
   ka.Tq_pad = g.Tq_pad;
   ka.eps = c.eps;
   ka.drop = c.drop;
+  // launches with few rows split each row's live units over S waves
+  auto split = [&](int tiles) {
+    const int64_t rows = (int64_t)2 * tiles * g.B * g.H;
+    return split_waves<T>(rows);
+  };
+  const dim3 qgrid((unsigned)(2 * g.nqt), (unsigned)(g.B * g.H)), kgrid((unsigned)(2 * g.nkt), (unsigned)(g.B * g.H));
   timer_begin(5, c.stream);
-  hipLaunchKernelGGL((dq_kernel<T, DP>), dim3((unsigned)(2 * g.nqt), (unsigned)(g.B * g.H)), dim3(64), 0, c.stream,
-                     ka);
+  switch (split(g.nqt)) {
+    case 4: hipLaunchKernelGGL((dq_kernel<T, DP, 4>), qgrid, dim3(256), 0, c.stream, ka); break;
+    case 2: hipLaunchKernelGGL((dq_kernel<T, DP, 2>), qgrid, dim3(128), 0, c.stream, ka); break;
+    default: hipLaunchKernelGGL((dq_kernel<T, DP, 1>), qgrid, dim3(64), 0, c.stream, ka);
+  }
   timer_end(5, c.stream);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   timer_begin(4, c.stream);
-  hipLaunchKernelGGL((dkdv_kernel<T, DP>), dim3((unsigned)(2 * g.nkt), (unsigned)(g.B * g.H)), dim3(64), 0, c.stream,
-                     ka);
+  switch (split(g.nkt)) {
+    case 4: hipLaunchKernelGGL((dkdv_kernel<T, DP, 4>), kgrid, dim3(256), 0, c.stream, ka); break;
+    case 2: hipLaunchKernelGGL((dkdv_kernel<T, DP, 2>), kgrid, dim3(128), 0, c.stream, ka); break;
+    default: hipLaunchKernelGGL((dkdv_kernel<T, DP, 1>), kgrid, dim3(64), 0, c.stream, ka);
+  }
   timer_end(4, c.stream);
   return hipGetLastError();
 }

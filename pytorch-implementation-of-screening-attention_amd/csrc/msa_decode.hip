@@ -380,9 +380,9 @@ __global__ __launch_bounds__(64) void selftest_kernel(const float* a16, const fl
     fb[e] = (bf16)b16[(8 * half + e) * 32 + l32];    // B[k][n=l32]
   }
   f32x16 c = {};
-  c = Mma<bf16>::mma(fa, fb, c);
+  c = Mma<bf16>::mma_ng(fa, fb, c);  // fa and fb are not written again
   f32x16 c2 = {};
-  c2 = Mma<float>::mma(a2[l32 * 2 + half], b2[half * 32 + l32], c2);
+  c2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a2[l32 * 2 + half], b2[half * 32 + l32], c2, 0, 0, 0);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = 8 * (r / 4) + 4 * half + (r % 4);

@@ -39,17 +39,13 @@ constexpr int kUnit = 32;  // rows of a query unit and of a key unit (live-unit 
 // The unguarded D=32 bf16 dq kernel shows a v_mov_b64 refilling SrcA one
 // instruction after such a chained v_mfma_f32_32x32x16_bf16.  Measured on an
 // MI355X: 2 and 4 wait states of padding still corrupted the product, 8 did
-// not.  After every MFMA group an s_nop block that takes A and B as read-write
-// operands keeps those registers from being reused until 16 wait states have
+// not.  After every MFMA group an s_nop block that takes A and B as operands
+// keeps those registers from being reused until 16 wait states have
 // passed.  The MFMA pipe is busy far longer than that per instruction, so
 // back-to-back MFMA throughput is unchanged.
 // ---------------------------------------------------------------------------
 template <typename T> struct Mma;
 
-template <typename F>
-__device__ inline void guard_mfma_sources(F& a, F& b) {
-  asm volatile("s_nop 7\n\ts_nop 7" : "+v"(a), "+v"(b));
-}
 // Group form: after a run of unguarded MFMAs (mma_ng), one s_nop block that
 // takes every A/B fragment of the run as a read-write operand.  The asm must
 // follow each MFMA that reads those registers (write-after-read order), so
@@ -84,16 +80,34 @@ __device__ inline void guard_frags(F (&f)[16]) {
                "+v"(f[14]), "+v"(f[15]));
 }
 
+// After a run of MFMAs (mma_ng) that ends in accumulator c: one block that
+// reads every A/B fragment of the run, so their registers stay allocated until
+// it, and c, which orders it after the run.  2-byte types wait 16 states in
+// it; fp32, whose 16-pass steps read later than that covers, waits for the
+// product itself by reading one of its registers.  guard_keep adds further
+// fragments of the same run.
+template <typename F, int N>
+__device__ inline void guard_keep(const F (&f)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; k += 2) asm volatile("" ::"v"(f[k]), "v"(f[k + 1]));
+}
+template <typename F, int N>
+__device__ inline void guard_run(const F (&f)[N], const f32x16& c) {
+  if constexpr (__is_same(F, f32x4)) {
+    const int x = __builtin_amdgcn_readfirstlane(__float_as_int(c[15]));
+#pragma unroll
+    for (int k = 0; k < N; k += 2) asm volatile("" ::"v"(f[k]), "v"(f[k + 1]), "s"(x));
+  } else {
+    asm volatile(MSA_NOP16 ::"v"(c[15]));
+    guard_keep(f);
+  }
+}
+
 template <> struct Mma<bf16> {
   static constexpr int KS = 16;
   static constexpr int PER = 8;
   typedef bf16x8 frag;
-  __device__ static inline f32x16 mma(frag a, frag b, f32x16 c) {
-    const f32x16 d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-    guard_mfma_sources(a, b);
-    return d;
-  }
-  // Unguarded: the caller guards every A/B fragment with guard_frags.
+  // Unguarded: the caller guards every A/B fragment with guard_run.
   __device__ static inline f32x16 mma_ng(frag a, frag b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
@@ -116,11 +130,6 @@ template <> struct Mma<f16> {
   static constexpr int KS = 16;
   static constexpr int PER = 8;
   typedef f16x8 frag;
-  __device__ static inline f32x16 mma(frag a, frag b, f32x16 c) {
-    const f32x16 d = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    guard_mfma_sources(a, b);
-    return d;
-  }
   __device__ static inline f32x16 mma_ng(frag a, frag b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }
@@ -136,32 +145,85 @@ template <> struct Mma<f16> {
 };
 
 // Where a per-row factor 1/|x| enters a product whose other operand is
-// packed to the input type.  bf16 (8 exponent bits) folds it into the pair
-// weights (alpha*m/|v|, ds/|k|, ds/|q|) and keeps the raw rows exact.  fp16
-// has 5 exponent bits: a weight times 1/|x| overflows to inf for rows shorter
-// than about 1.5e-5 (a zero row gives 1/eps = 1e8, then inf * 0 = NaN), so
-// the fp16 kernels scale the transposed rows instead (x^ = x/|x|, at most 1
-// in magnitude) and the weights stay at most 2r|dP|.
+// packed to the input type.  bf16 (8 exponent bits) and fp32 fold it into the
+// pair weights (alpha*m/|v|, ds/|k|, ds/|q|) and keep the raw rows exact.
+// fp16 has 5 exponent bits: a weight times 1/|x| overflows to inf for rows
+// shorter than about 1.5e-5 (a zero row gives 1/eps = 1e8, then inf * 0 =
+// NaN).  There 1/|x| = c w with c a power of two and w in [1/2, 1]: the rows
+// take c, which only moves their exponent, and the weights take w.
 template <typename T>
-constexpr bool kScaleRowsNotWeights = sizeof(T) == 2 && !__is_same(T, bf16);
+constexpr bool kPow2Rows = sizeof(T) == 2 && !__is_same(T, bf16);
 
-template <> struct Mma<float> {
-  static constexpr int KS = 2;
-  static constexpr int PER = 1;
-  typedef float frag;
-  __device__ static inline f32x16 mma(frag a, frag b, f32x16 c) {
-    const f32x16 d = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-    guard_mfma_sources(a, b);
-    return d;
+// The split of a row factor f = 1/|x| (0 for masked rows): w <= 1 and c = c1 c2,
+// each a power of two in fp16's normal range.  c2 is 1 except for rows
+// shorter than 2^-15; a zero row (f = 1/eps, past c's range) has w = 1 and
+// contributes its zeros whatever w is.  |x| > 2^14 leaves c at 2^-14.
+struct Pow2Split {
+  float w, c1, c2;
+  __device__ explicit Pow2Split(float f) {
+    const float c = __int_as_float((__float_as_int(f) & 0x7f800000) + 0x00800000);
+    c1 = fminf(fmaxf(c, 6.103515625e-5f), 32768.0f);                    // 2^-14 .. 2^15
+    c2 = fminf(fmaxf(c * 3.0517578125e-5f, 1.0f), 32768.0f);             // c 2^-15
+    w = fminf(f * recip(c1) * recip(c2), 1.0f);
   }
-  __device__ static inline f32x16 mma_ng(frag a, frag b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static inline frag load(const float* p) { return *p; }
-  __device__ static inline frag zero() { return 0.0f; }
-  __device__ static inline float get(const frag& f, int) { return f; }
-  __device__ static inline frag pack(const f32x16& c, int r0) { return c[r0]; }
+  __device__ static inline float recip(float p) { return __int_as_float(0x7f000000 - __float_as_int(p)); }  // 1/2^e
 };
+
+// fp32: a fragment is four v_mfma_f32_32x32x2_f32 steps, step e contracting the
+// lanes' slot e (half 0: column 8ks + e, half 1: column 8ks + 4 + e), so a
+// lane's slots are 16 contiguous bytes of its row as for the 2-byte types.
+template <> struct Mma<float> {
+  static constexpr int KS = 8;
+  static constexpr int PER = 4;
+  typedef f32x4 frag;
+  __device__ static inline f32x16 mma_ng(const frag& a, const frag& b, f32x16 c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], c, 0, 0, 0);
+    return c;
+  }
+  __device__ static inline frag load(const float* p) { return *reinterpret_cast<const frag*>(p); }
+  __device__ static inline frag zero() { return frag{0.0f, 0.0f, 0.0f, 0.0f}; }
+  __device__ static inline float get(const frag& f, int e) { return f[e]; }
+  __device__ static inline frag pack(const f32x16& c, int r0) { return frag{c[r0], c[r0 + 1], c[r0 + 2], c[r0 + 3]}; }
+};
+
+// Waves per SIMD the live and dq passes are register-budgeted for, by a row's bytes.
+template <typename T, int DP>
+constexpr int unit_waves() { return sizeof(T) * DP <= 128 ? 3 : (sizeof(T) * DP <= 256 ? 2 : 1); }
+
+// The 32x32 product of two units' row fragments.  fp32 keeps one accumulator
+// per slot: four chains of D/8 roundings over quarter sums instead of one of
+// D/2 over the whole, and four independent MFMA chains; with `lo`, the
+// rounding error of the last addition is kept too (two-sum).  Pairs just above
+// the threshold magnify an error of s by 2r/a, so s is formed more exactly
+// than the rest; the live, dq and dK/dV passes all form it here, in one order.
+template <typename T, int N>
+__device__ inline f32x16 unit_product(const typename Mma<T>::frag (&a)[N], const typename Mma<T>::frag (&b)[N],
+                                      f32x16* lo = nullptr) {
+  f32x16 z;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) z[r] = 0.0f;
+  if constexpr (sizeof(T) == 2) {
+#pragma unroll
+    for (int ks = 0; ks < N; ++ks) z = Mma<T>::mma_ng(a[ks], b[ks], z);
+  } else {
+    f32x16 c[4] = {z, z, z, z};
+#pragma unroll
+    for (int ks = 0; ks < N; ++ks)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) c[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[ks][e], b[ks][e], c[e], 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float x = c[0][r] + c[1][r], y = c[2][r] + c[3][r];
+      z[r] = x + y;
+      if (lo != nullptr) {
+        const float v = z[r] - x;
+        (*lo)[r] = (x - (z[r] - v)) + (y - v);
+      }
+    }
+  }
+  return z;
+}
 
 // Row permutation applied when a lane loads row (l%32) of an A operand whose
 // product lands in a C block that is later consumed as the B operand of a
@@ -191,49 +253,20 @@ __device__ inline int rowof(int r, int half) { return 16 * (r >> 3) + 8 * half +
 template <typename T>
 __device__ inline int tcol(int m) {
   if constexpr (sizeof(T) == 2) return perm_row(m);                 // 16*(m/16) + 8*((m>>2)&1) + ...
-  else return 8 * (m >> 3) + 2 * (m & 3) + ((m >> 2) & 1);
+  else return m;
 }
 // Fragment slot (ks, e) that holds, in the same lane, the column that register
 // r of C block dblk covers when the block's rows are tcol-ordered columns.
 template <typename T>
 __device__ constexpr int creg_ks(int dblk, int r) {
   if constexpr (sizeof(T) == 2) return 2 * dblk + (r >> 3);   // column 32*dblk + 16*(r/8) + 8*half + r%8
-  else return 16 * dblk + 4 * (r >> 2) + (r & 3);             // column 32*dblk + 8*(r/4) + 2*(r%4) + half
+  else return 4 * dblk + (r >> 2);                            // column 32*dblk + 8*(r/4) + 4*half + r%4
 }
 template <typename T>
 __device__ constexpr int creg_e(int r) {
   if constexpr (sizeof(T) == 2) return r & 7;
-  else return 0;
+  else return r & 3;
 }
-// Slice c of the permutation (k-step c of a 32-column block; it does not
-// depend on the block): slot e of lane l is 1 iff KS*c + PER*(l/32) + e ==
-// tcol(l%32).
-template <typename T>
-__device__ inline typename Mma<T>::frag ident_frag(int c, int lane) {
-  using M = Mma<T>;
-  const int l32 = lane & 31, half = lane >> 5;
-  const int want = tcol<T>(l32);
-  f32x16 t;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) t[e] = (e < M::PER && M::KS * c + M::PER * half + e == want) ? 1.0f : 0.0f;
-  return M::pack(t, 0);
-}
-// out[dblk] = (X I)[:, 32*dblk .. 32*dblk+31] with unguarded MFMAs: the
-// caller guards x and id (guard_frags) before they can be overwritten.
-template <typename T, int DP>
-__device__ inline void transpose_rows(const typename Mma<T>::frag (&x)[DP / Mma<T>::KS],
-                                      const typename Mma<T>::frag (&id)[32 / Mma<T>::KS], f32x16 (&out)[DP / 32]) {
-  using M = Mma<T>;
-  constexpr int NC = 32 / M::KS;
-#pragma unroll
-  for (int dblk = 0; dblk < DP / 32; ++dblk) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) out[dblk][r] = 0.0f;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) out[dblk] = M::mma_ng(x[dblk * NC + c], id[c], out[dblk]);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Screening math for one (query i, key j) pair.
 // ---------------------------------------------------------------------------
@@ -259,9 +292,9 @@ struct HeadParams {
 __device__ inline HeadParams head_params_rw(float r, float w, bool causal) {
   HeadParams p;
   p.r = r;
-  p.w = w;
+  p.w = fminf(w, 1e30f);  // an infinite window: the mask is 1 (and no inf * 0 in it)
   p.iw = 1.0f / p.w;
-  const float c = ceilf(p.w);
+  const float c = ceilf(w);
   p.wc = !(c > 0.0f) ? 0 : (c > 1073741824.0f ? 1073741824 : (int)c);
   p.thr = 1.0f - 1.0f / p.r - 1e-5f;
   p.wsh = causal ? 0 : p.wc - 1;
@@ -298,22 +331,9 @@ __device__ inline void for_each_set(uint32_t pm, Fn&& fn) {
   }
 }
 
-// cos(pi x) and sin(pi x) for |x| <= 1 (x clamped there), branch-free and
-// without a library call: with y = |x| and t = min(y, 1 - y) in [0, 1/2],
-// cos(pi y) = +-cos(pi t) (minus for y > 1/2) and sin(pi y) = sin(pi t); the
-// Taylor series of cos(pi t) and sin(pi t) to t^12 and t^13 are within
-// 6.4e-9 and 6.7e-10 of them on [0, 1/2] (next terms pi^14 t^14/14! and
-// pi^15 t^15/15!), below fp32 rounding.  Coefficients (-1)^k pi^2k/(2k)!
-// and (-1)^k pi^(2k+1)/(2k+1)!, evaluated by Horner's rule in t^2.
-__device__ inline float cospi_poly(float u) {  // u = t^2
-  float c = 0.001929574309403922f;
-  c = fmaf(c, u, -0.02580689139001405f);
-  c = fmaf(c, u, 0.23533063035889312f);
-  c = fmaf(c, u, -1.3352627688545893f);
-  c = fmaf(c, u, 4.058712126416768f);
-  c = fmaf(c, u, -4.934802200544679f);
-  return fmaf(c, u, 1.0f);
-}
+// sin(pi t) for t in [0, 1/2]: the Taylor series to t^13 is within 6.7e-10
+// (next term pi^15 t^15/15!), below fp32 rounding.  Coefficients (-1)^k
+// pi^(2k+1)/(2k+1)!, evaluated by Horner's rule in u = t^2.
 __device__ inline float sinpi_poly(float t, float u) {  // u = t^2
   float c = 0.00046630280576761234f;
   c = fmaf(c, u, -0.007370430945714348f);
@@ -325,40 +345,28 @@ __device__ inline float sinpi_poly(float t, float u) {  // u = t^2
   return c * t;
 }
 // Soft mask m = (cos(pi dd/w) + 1)/2 (attention.py:114) for an in-window
-// distance (|dd| < w, so y = |dd|/w < 1); out of the window the value is
-// finite and the caller masks it.  For y <= 1/2, m = 1/2 + cos(pi y)/2 (both
-// terms at least 0: no cancellation).  Past 1/2, m falls to 0 at the window's
-// edge and that form would cancel, and y = |dd| (1/w) would carry the
-// rounding of 1/w into 1 - y; there m = sin^2(pi t/2) with t = 1 - y formed
-// as (w - |dd|) / w, whose numerator is exact in fp32 (w/2 <= |dd| <= w:
-// Sterbenz), so m keeps a few ulps of relative accuracy down to the last
-// in-window distance.  t also gives sin(pi y) = sin(pi t) for dm/dw.
-struct MaskArg {
-  float y, t;  // |dd|/w, and min(y, 1 - y) with 1 - y = (w - |dd|)/w
-  bool far;    // y > 1/2
-};
-__device__ inline MaskArg mask_arg(int dd, float w, float iw) {
-  MaskArg a;
-  const float ad = fabsf((float)dd);
-  a.y = fminf(ad * iw, 1.0f);
-  a.far = a.y > 0.5f;
-  a.t = a.far ? fmaxf((w - ad) * iw, 0.0f) : a.y;
-  return a;
+// distance (|dd| < w); out of the window the value is finite and the caller
+// masks it.  m = sin^2(pi z) with z = (w - |dd|)/(2w) in [0, 1/2]: one
+// polynomial, and near the window's end, where m falls to 0 and the cosine
+// form would cancel, w - |dd| is exact in fp32 (w/2 <= |dd| <= w: Sterbenz),
+// so m keeps a few ulps of relative accuracy down to the last distance.
+__device__ inline float mask_root(int dd, float w, float iw) {
+  const float z = fmaxf((w - fabsf((float)dd)) * iw * 0.5f, 0.0f);
+  return sinpi_poly(z, z * z);
 }
-__device__ inline float mask_of(const MaskArg& a) {
-  const float z = 0.5f * a.t;  // sin(pi t/2) for the far half
-  const float sz = sinpi_poly(z, z * z);
-  const float c = cospi_poly(a.t * a.t);
-  return a.far ? sz * sz : 0.5f + 0.5f * c;
+__device__ inline float mask_fast(int dd, float w, float iw) {
+  const float s = mask_root(dd, w, iw);
+  return s * s;
 }
-__device__ inline float mask_fast(int dd, float w, float iw) { return mask_of(mask_arg(dd, w, iw)); }
 // The same mask and dm/dw = (pi/2) dd sin(pi dd/w) / w^2 (the w-derivative
-// of (cos(pi (j-i)/w) + 1)/2, attention.py:114).
+// of (cos(pi (j-i)/w) + 1)/2, attention.py:114), with sin(pi y) = 2 sin(pi y/2)
+// cos(pi y/2) and cos(pi y/2) = sin(pi (1 - y)/2), the mask's root: both
+// factors keep their relative accuracy where they fall to 0.
 __device__ inline void mask_fast_dw(int dd, float w, float iw, float& m, float& dm) {
-  const MaskArg a = mask_arg(dd, w, iw);
-  m = mask_of(a);
-  const float sn = copysignf(sinpi_poly(a.t, a.t * a.t), (float)dd);
-  dm = (0.5f * 3.14159265358979f) * (float)dd * sn * iw * iw;
+  const float s = mask_root(dd, w, iw);
+  const float x = (float)dd * iw, y = fminf(0.5f * fabsf(x), 0.5f);
+  m = s * s;
+  dm = 3.14159265358979f * fabsf(x) * iw * s * sinpi_poly(y, y * y);
 }
 
 // Branch-free in-window test on the integer distance dd = i - j.
@@ -386,6 +394,28 @@ __device__ inline void unit_mask_table(float* mt, float* mdt, int dmin, const He
 
 // Trim-and-square pre-square value a = 1 - r (1 - s)  (attention.py:90).
 __device__ inline float trim(float s, float r) { return 1.0f - r * (1.0f - s); }
+
+// s = (acc + lo) f of an fp32 product's register, f the factor 1/|x| of one
+// side: acc becomes the rounded product and lo its error (2-byte types: no lo).
+template <typename T>
+__device__ inline void scale_pair(f32x16& acc, f32x16& lo, int r, float f) {
+  const float t = acc[r] * f;
+  if constexpr (sizeof(T) == 4) lo[r] = fmaf(lo[r], f, fmaf(acc[r], f, -t));
+  acc[r] = t;
+}
+// alpha's root max(1 - r(1 - s), 0) of s = (acc + lo) f, f the other side's
+// factor.  2-byte types: one fma with rf = r f and the clamp to [0, 1] (a
+// modifier of it) in place of the multiply and trim; the rounding, 2^-24 of 1
+// and of r, is that of the longer form.
+template <typename T>
+__device__ inline float pair_root(float acc, float lo, float f, float rf, float r) {
+  if constexpr (sizeof(T) == 4) {
+    const float s = acc * f;
+    return fmaxf(fmaf(r, fmaf(lo, f, fmaf(acc, f, -s)), trim(s, r)), 0.0f);
+  } else {
+    return __builtin_amdgcn_fmed3f(fmaf(acc, rf, 1.0f - r), 0.0f, 1.0f);
+  }
+}
 
 // max(x[l], x[l ^ 32]) in every lane (as half_sum, with max).
 __device__ inline float half_max(float x) {
@@ -490,9 +520,9 @@ __device__ inline void store_creg_row(T* row, int D, int half, Fn fn) {
 #pragma unroll
     for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int d = 32 * dblk + 8 * (r >> 2) + 2 * (r & 3) + half;
-        if (d < D) row[d] = fn(dblk, r);
+      for (int g = 0; g < 4; ++g) {
+        const int d0 = 32 * dblk + 8 * g + 4 * half;
+        if (d0 < D) store4(row + d0, fn(dblk, 4 * g), fn(dblk, 4 * g + 1), fn(dblk, 4 * g + 2), fn(dblk, 4 * g + 3));
       }
   }
 }
@@ -521,6 +551,20 @@ __device__ inline float inv_len(float ss, float eps) {
   return fminf(__builtin_amdgcn_rsqf(ss), __builtin_amdgcn_rcpf(eps));
 }
 
+// The same for a row of type T's unit kernels.  fp32 rows take one Newton step
+// more (half an ulp instead of one), which the pairs just above the threshold
+// need; zero and infinite lengths keep the plain value.
+template <typename T>
+__device__ inline float inv_len_of(float ss, float eps) {
+  if constexpr (sizeof(T) == 2) {
+    return inv_len(ss, eps);
+  } else {
+    const float y = __builtin_amdgcn_rsqf(ss);
+    const float z = fmaf(0.5f * y, fmaf(-ss * y, y, 1.0f), y);
+    return fminf(ss > 0.0f && ss < INFINITY ? z : y, __builtin_amdgcn_rcpf(eps));
+  }
+}
+
 // Sum of products of two operand fragments in fp32: v_dot2c_f32_bf16 (two
 // exact bf16 products per instruction) for bf16, a plain product for fp32.
 __device__ inline float frag_dot(const bf16x8& a, const bf16x8& b, float acc) {
@@ -542,7 +586,24 @@ __device__ inline float frag_dot(const f16x8& a, const f16x8& b, float acc) {
   }
   return acc;
 }
-__device__ inline float frag_dot(float a, float b, float acc) { return acc + a * b; }
+// Sum of products of two fragment rows (this lane's slots).  fp32 keeps one
+// chain per slot: D/8 roundings each instead of D/2 in one.
+template <typename T, int N>
+__device__ inline float row_dot(const typename Mma<T>::frag (&a)[N], const typename Mma<T>::frag (&b)[N]) {
+  if constexpr (sizeof(T) == 2) {
+    float s = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < N; ++ks) s = frag_dot(a[ks], b[ks], s);
+    return s;
+  } else {
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ks = 0; ks < N; ++ks)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] = fmaf(a[ks][e], b[ks][e], s[e]);
+    return (s[0] + s[1]) + (s[2] + s[3]);
+  }
+}
 
 // An operand row kept in its storage type: the lane's NKS fragments (slots
 // d = KS*ks + PER*half + e), converted to fp32 only where arithmetic needs it.
@@ -566,13 +627,8 @@ struct PRow {
       if (!(ok && KS * ks + PER * half < D)) f[ks] = M::zero();
   }
   __device__ inline float get(int ks, int e) const { return M::get(f[ks], e); }
-  __device__ inline float dot(const PRow& o) const {
-    float s = 0.0f;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) s = frag_dot(f[ks], o.f[ks], s);
-    return half_sum(s);
-  }
-  __device__ inline float inv_norm(float eps) const { return inv_len(dot(*this), eps); }
+  __device__ inline float dot(const PRow& o) const { return half_sum(row_dot<T>(f, o.f)); }
+  __device__ inline float inv_norm(float eps) const { return inv_len_of<T>(dot(*this), eps); }
   // this <- a*this + b*o, rounded to T
   __device__ inline void axpby(float a, float b, const PRow& o) {
 #pragma unroll
@@ -598,17 +654,10 @@ __device__ inline void read_row_scales(const float* sc, int half, float (&o)[16]
     }
 }
 
-// fp16 row scaling of an identity-MFMA transpose: c holds the raw rows
-// exactly in fp32 (products with 1, sums with 0), register r row
-// 16*(r/8) + 8*half + r%8, and each register takes its row's factor in fp32;
-// the operand pack then rounds once to fp16.  The same value as scaling the
-// row registers before the transpose, at one multiply per register instead
-// of a convert, multiply and convert per element.
-__device__ inline void scale_rows_fp32(f32x16& c, const float* sc, int half) {
-  float f[16];
-  read_row_scales(sc, half, f);
-#pragma unroll
-  for (int r = 0; r < 16; ++r) c[r] *= f[r];
+// Multiplies column fragment c's slots (rows rowof(8c + e, half)) by the rows'
+// powers of two, from an LDS vector of 32 fp16 values in row order.
+__device__ inline void scale_slots(f16x8& f, const f16* sc, int c, int half) {
+  f *= *reinterpret_cast<const f16x8*>(sc + 16 * c + 8 * half);
 }
 
 // Waits until at most N of this wave's vector memory operations (loads,
@@ -632,12 +681,129 @@ __device__ inline void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" :::
 //          and on {4..7, 12..15}, and on the even and the odd rows of 0..15;
 //   CPR>=16: (b1, b3, b0^b2, b0) is also one-to-one on all of 0..15.
 template <int CPR>
-__device__ inline int lds_swz(int R) {
+__device__ constexpr int lds_swz(int R) {
   const int b0 = R & 1, b1 = (R >> 1) & 1, b2 = (R >> 2) & 1, b3 = (R >> 3) & 1;
   if constexpr (CPR == 4) return (b1 ^ b2) | (b3 << 1);
   else if constexpr (CPR == 8) return b1 | (b3 << 1) | ((b0 ^ b2) << 2);
   else return b1 | (b3 << 1) | ((b0 ^ b2) << 2) | (b0 << 3);
 }
+
+// ---------------------------------------------------------------------------
+// A 32-row unit of a (B,T,H,D) tensor staged in a wave's own LDS.  The rows
+// come by direct DMA, each instruction moving whole rows (1 KiB: 8 rows of
+// 128 bytes), and are then read in both orders an MFMA takes them: as row
+// fragments (lane -> row perm_row(l%32)) and, transposed, as column fragments
+// (lane -> column, slots -> rows) by ds_read_b64_tr_b16 (2-byte types) or
+// plain 4-byte reads (fp32).  Loaded straight into operand registers instead,
+// every load instruction touches 32 rows (of fp32 4 bytes each), the next
+// unit's rows occupy registers, and each transpose costs identity MFMAs and
+// repacking.  Measured, live / dq / dK/dV: B=4, T=8192, H=8, D=64 bf16 with
+// every unit live 716 / 712 / 702 -> 504 / 693 / 478 us; B=2, T=1500 fp32
+// 207 / 370 / 440 -> 97 / 125 / 137 us.
+// Chunks of 16 bytes are XOR-swizzled within their row (lds_swz): the DMA
+// writes linearly, so each lane fetches the chunk that belongs at its place.
+// lds_swz is linear over the row's bits, so offsets of other rows, steps and
+// column blocks are one XOR with a constant away from the lane's base.
+// ---------------------------------------------------------------------------
+// LDS destinations keep their address space: with the shared array known the
+// compiler sees that the pass's other LDS arrays do not alias it (it waits for
+// a copy in flight before any LDS read that might).
+typedef __attribute__((address_space(3))) char LdsChar;
+template <typename T, int DP>
+struct UnitTile {
+  using M = Mma<T>;
+  using frag = typename M::frag;
+  static constexpr int ROWB = DP * (int)sizeof(T), CPR = ROWB / 16, BYTES = kUnit * ROWB;
+  static constexpr int NI = BYTES / 1024;  // DMA instructions per unit
+  static constexpr int RPI = 1024 / ROWB;  // rows per DMA instruction
+  static constexpr int NKS = DP / M::KS, NDH = DP / 32, NC = 32 / M::KS;
+  __device__ static constexpr int swz(int R) { return lds_swz<CPR>(R); }
+
+  // The lane's place in the DMA of a tensor with rows `stb` bytes apart.
+  struct Source {
+    const char* base;  // row 0 of the head
+    uint32_t stb;
+    int rows;          // rows of the tensor (rows past them read the last one)
+    uint32_t lrow, cb;
+    uint32_t cmask;    // D = 16 of DP = 32: chunks past D re-read the row's first ones
+    __device__ Source(const T* head, int64_t st, int rows_, int D, int lane)
+        : base((const char*)head), stb((uint32_t)(st * (int64_t)sizeof(T))), rows(rows_),
+          lrow((uint32_t)(lane / CPR)), cb((uint32_t)((lane % CPR) ^ swz(lane / CPR)) << 4),
+          cmask(DP == 32 && D < DP ? (uint32_t)(D * (int)sizeof(T) - 1) : 0xffffffffu) {}
+    // Starts the copy of unit u to LDS address `lds` (wave-uniform; RPI rows, 1 KiB, an
+    // instruction).  Row offsets stay below 2^32 bytes: 64 rows span less.
+    __device__ inline void issue(LdsChar* lds, int u) const {
+      const char* ub = base + (int64_t)u * kUnit * stb;
+      const int last = rows - 1 - u * kUnit;
+      if (last >= kUnit - 1) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) dma(ub + (int64_t)(i * RPI) * stb + (uint32_t)(lrow * stb + chunk(i)), lds, i);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int r = i * RPI + (int)lrow;
+          dma(ub + (uint32_t)((uint32_t)(r < last ? r : last) * stb + chunk(i)), lds, i);
+        }
+      }
+    }
+    __device__ inline uint32_t chunk(int i) const {
+      const uint32_t c = cb ^ (uint32_t)(swz((i * RPI) & 15) << 4);
+      return DP == 32 ? c & cmask : c;
+    }
+    __device__ static inline void dma(const char* src, LdsChar* lds, int i) {
+      __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                       (void __attribute__((address_space(3)))*)(lds + i * 1024), 16, 0, 0);
+    }
+  };
+
+  // Row fragments: lane -> row perm_row(l%32), slots -> columns KS*ks + PER*half + e.
+  __device__ static inline uint32_t row_base(int lane) {
+    const int R = perm_row(lane & 31);
+    return (uint32_t)(R * ROWB + (((lane >> 5) ^ swz(R)) << 4));
+  }
+  __device__ static inline frag row_frag(const char* tile, uint32_t rb, int ks) {
+    return *reinterpret_cast<const frag*>(tile + (rb ^ (uint32_t)(ks << 5)));
+  }
+  // Column fragments: lane -> column 32*dblk + tcol(l%32), slots -> rows
+  // rowof(PER*c + e, half), the rows of a C block's registers PER*c + e.
+  __device__ static inline uint32_t col_base(int lane) {
+    const int half = lane >> 5, l32 = lane & 31;
+    if constexpr (sizeof(T) == 2) {
+      // a 16-lane group transposes 4 rows x 16 columns: lane 4k + q gives row
+      // k's 4 columns 16gg + 8(q&1) + 4(q>>1), and lane i takes column i
+      const int k = (lane & 15) >> 2, q = lane & 3, gg = l32 >> 4, R = 8 * half + k;
+      return (uint32_t)(R * ROWB + (((2 * gg + (q & 1)) ^ swz(R)) << 4) + 8 * (q >> 1));
+    } else {
+      const int R = 8 * half;
+      return (uint32_t)(R * ROWB + (((l32 >> 2) ^ swz(R)) << 4) + 4 * (l32 & 3));
+    }
+  }
+  __device__ static inline frag col_frag(const char* tile, uint32_t cbase, int dblk, int c) {
+    if constexpr (sizeof(T) == 2) {
+      typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
+      typedef __attribute__((__vector_size__(8 * sizeof(short)))) short s16x8;
+      s16x8 v;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const char* p = tile + (cbase ^ (uint32_t)((swz(4 * j) ^ (4 * dblk)) << 4)) + (16 * c + 4 * j) * ROWB;
+        const s16x4 x =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)const_cast<char*>(p));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * j + e] = x[e];
+      }
+      return __builtin_bit_cast(frag, v);
+    } else {
+      frag v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int R = 4 * (c & 1) + e;
+        v[e] = *reinterpret_cast<const float*>(tile + (cbase ^ (uint32_t)((swz(R) ^ (8 * dblk)) << 4)) +
+                                               (16 * (c >> 1) + R) * ROWB);
+      }
+      return v;
+    }
+  }
+};
 
 // Set bits lo..hi of one bitmap row (position u = bit u%32 of word u/32),
 // visited in increasing order.  Lane l holds word w0 + l, so one load round

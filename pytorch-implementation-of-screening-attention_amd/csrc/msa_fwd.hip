@@ -772,44 +772,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // ---------------------------------------------------------------------------
 // Live units.  One wave (a 64-thread block) per query unit: 32 consecutive
 // queries of one head, lane -> query i = 32*qu + l%32.  The wave walks its
-// row of the live-unit bitmap; for each live key unit (32 keys) it loads the
-// raw K and V rows straight from global memory as MFMA operands, the next
-// unit's loads in flight while the current one is computed: S^T = K Q^T on
-// the raw values (exact products, as the backward forms it) scaled by
-// 1/|k_j| in fp32, alpha*m (attention.py:92-119) with 1/|v_j| folded in
-// (fp16: into the V rows), and H^T += V^T P^T with V^T from an identity MFMA
-// on the raw V rows.  The
-// epilogue applies TanhNorm (norm.py:23-25) and writes y in (B,T,H,D) and |h|
-// per row.  Units with no live key unit get y = 0, |h| = 0.
-// S > 1 (launches with at most kLiveSplitWaves / S rows, D <= 64): S waves
-// per row in one block, wave w taking the row's live units w, w+S, ...; waves
-// 1..S-1 hand their partial H^T to wave 0 through LDS, which adds them in
-// wave order (fixed, so results repeat bitwise) and runs the epilogue.
+// row of the live-unit bitmap; each live key unit's raw K and V rows (32 keys)
+// are staged in the wave's own LDS (UnitTile), the next unit's copies in
+// flight while the current one is computed: S^T = K Q^T on the raw values
+// (exact products, as the backward forms it) scaled by 1/|k_j| in fp32,
+// alpha*m (attention.py:92-119) with 1/|v_j| folded in (fp16: its power of two
+// into the V columns), and H^T += V^T P^T with V^T read transposed from the
+// staged rows.  The epilogue applies TanhNorm (norm.py:23-25) and writes y in
+// (B,T,H,D) and |h| per row.  Units with no live key unit get y = 0, |h| = 0.
+// S > 1 (launches with few rows): S waves per row in one block, wave w taking
+// the row's live units w, w+S, ...; waves 1..S-1 hand their partial H^T to
+// wave 0 through LDS, which adds them in wave order (fixed, so results repeat
+// bitwise) and runs the epilogue.
 // ---------------------------------------------------------------------------
 template <typename T, int DP, int S>
-__global__ __launch_bounds__(64 * S)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && DP <= 64 ? 3 : (S > 1 ? (DP <= 32 ? 3 : 2) : 1))))
+__global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(unit_waves<T, DP>())))
 void fwd_live_kernel(FwdKArgs a) {
   using M = Mma<T>;
   using frag = typename M::frag;
   using R = PRow<T, DP>;
+  using U = UnitTile<T, DP>;
   constexpr int KS = M::KS, PER = M::PER, NKS = DP / KS, NDH = DP / 32, NC = 32 / KS;
   // per wave:
   __shared__ __attribute__((aligned(16))) float sk_w[S][32];  // 1/|k_j| (0 if padded or masked) of the current unit
-  __shared__ __attribute__((aligned(16))) float sv_w[S][32];  // 1/|v_j| of the current unit's key rows
+  __shared__ __attribute__((aligned(16))) float sv_w[S][32];  // 1/|v_j| of the current unit's key rows (fp16: its w)
   __shared__ float mt_w[S][64];  // soft-mask table of the current unit (unit_mask_table)
-  // own raw q operand fragments; with S > 1 the same bytes then take the
-  // wave's partial H^T for wave 0 (after the wave's last read of its q)
-  constexpr int kQshBytes = NKS * kWave * (int)sizeof(frag);
-  constexpr int kPartBytes = NDH * 16 * kWave * 4;
-  constexpr int kWaveBytes = S > 1 && kPartBytes > kQshBytes ? kPartBytes : kQshBytes;
-  __shared__ __attribute__((aligned(16))) char wbuf[S][kWaveBytes];
+  __shared__ __attribute__((aligned(16))) f16 sc_w[S][2][32];  // fp16: the V rows' powers of two (Pow2Split)
+  // the current unit's K and V rows; with S > 1 the bytes then take the
+  // wave's partial H^T for wave 0
+  __shared__ __attribute__((aligned(1024))) char stage[S][2 * U::BYTES];
+  static_assert(NDH * 16 * kWave * 4 <= 2 * U::BYTES, "the partial H^T fits the staged rows");
   const int lane = (int)(threadIdx.x & 63), half = lane >> 5, l32 = lane & 31;
   const int wave = S > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
   float* sk = sk_w[wave];
   float* sv = sv_w[wave];
   float* mt = mt_w[wave];
-  frag (&qsh)[NKS][kWave] = *reinterpret_cast<frag(*)[NKS][kWave]>(wbuf[wave]);
+  char* kt = stage[wave];
+  char* vt = kt + U::BYTES;
+  LdsChar* const kt_at = (LdsChar*)&stage[0][0] + wave * 2 * U::BYTES;
+  LdsChar* const vt_at = kt_at + U::BYTES;
   int qu, bh;
   float head_r, head_w;
   xcd_interleave_ranked(a.r, a.w, a.H, qu, bh, head_r, head_w);
@@ -844,34 +845,21 @@ void fwd_live_kernel(FwdKArgs a) {
     }
     return;
   }
+  // S > 1: this wave's first unit is the row's live unit number `wave`
+  for (int w = 0; w < wave && cur >= 0; ++w) cur = walk.next();
 
   // key row of this lane in unit u: 32u + perm_row(l32) (A-operand order)
   const int m = perm_row(l32);
-  const T* kg = (const T*)a.k + b * a.ks.sb + h * a.ks.sh;
-  const T* vg = (const T*)a.v + b * a.vs.sb + h * a.vs.sh;
-  // The lane's chunks (elements KS*ks + PER*half) of its raw K or V row of
-  // key unit u, from one row address and immediate offsets: a wave-uniform
-  // 64-bit unit base plus a 32-bit lane offset.  Rows past Tk read row Tk-1
-  // instead; their 1/|k| is 0 (as for masked keys), so they never pass the
-  // threshold and their P is exactly 0.  Only D = 16 < DP has chunks past D
-  // (they re-read chunk 0; vzero clears them).
-  auto load_rows = [&](const T* base, int64_t st, int u, frag (&f)[NKS]) {
-    const int r = u * kUnit + m < a.Tk ? m : a.Tk - 1 - u * kUnit;
-    const uint32_t off = (uint32_t)(((int64_t)r * st + PER * half) * (int64_t)sizeof(T));
-    const char* p = (const char*)(base + (int64_t)u * kUnit * st) + off;
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-      const int c = DP == 32 && KS * ks >= a.D ? 0 : KS * ks;
-      f[ks] = M::load((const T*)(p + c * (int)sizeof(T)));
-    }
-  };
-  auto load_k = [&](int u, frag (&f)[NKS]) { load_rows(kg, a.ks.st, u, f); };
-  auto load_v = [&](int u, frag (&f)[NKS]) { load_rows(vg, a.vs.st, u, f); };
-  // 1/|k| is 0 for keys past Tk and for masked keys
-  auto key_ok = [&](int u) {
+  const typename U::Source ksrc((const T*)a.k + b * a.ks.sb + h * a.ks.sh, a.ks.st, a.Tk, a.D, lane);
+  const typename U::Source vsrc((const T*)a.v + b * a.vs.sb + h * a.vs.sh, a.vs.st, a.Tk, a.D, lane);
+  const uint32_t rb = U::row_base(lane), cb = U::col_base(lane);
+  // 1/|k| is 0 for keys past Tk and for masked keys, so they never pass the
+  // threshold and their P is exactly 0
+  auto key_mask = [&](int u) -> unsigned {  // the mask byte, tested when the unit is computed
     const int j = u * kUnit + m;
-    return j < a.Tk && !(a.kpm != nullptr && a.kpm[(int64_t)b * a.Tk + j] != 0);
+    return a.kpm != nullptr && j < a.Tk ? a.kpm[(int64_t)b * a.Tk + j] : 0u;
   };
+  // D = 16: the staged columns past D repeat the first ones
   auto vzero = [&](frag (&f)[NKS]) {
     if constexpr (DP == 32) {
 #pragma unroll
@@ -879,29 +867,19 @@ void fwd_live_kernel(FwdKArgs a) {
         if (KS * ks >= a.D) f[ks] = M::zero();
     }
   };
-  // S > 1: this wave's first unit is the row's live unit number `wave` (a
-  // wave left without one loads the row's first unit's rows and skips the
-  // loop)
-  const int first = cur;
-  for (int w = 0; w < wave && cur >= 0; ++w) cur = walk.next();
-  // own queries as raw B operands (lane -> query), kept in LDS and read back
-  // per unit (the registers go to the unit rows), and 1/|q_i|; their loads
-  // go first, the first unit's behind them
-  float iq;
-  frag kc[NKS], vc[NKS];
-  bool kok;
-  {
-    R qr;
-    qr.load((const T*)a.q + b * a.qs.sb + (int64_t)(valid ? i : 0) * a.qs.st + h * a.qs.sh, valid, a.D, half);
-    const int u0 = cur >= 0 ? cur : first;
-    load_k(u0, kc);
-    load_v(u0, vc);
-    kok = key_ok(u0);
-    iq = qr.inv_norm(a.eps);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) qsh[ks][lane] = qr.f[ks];
+  // own queries as raw B operands (lane -> query) and 1/|q_i|; their loads go
+  // first, the first unit's copies behind them
+  R qr;
+  unsigned kmask = 0u;
+  qr.load((const T*)a.q + b * a.qs.sb + (int64_t)(valid ? i : 0) * a.qs.st + h * a.qs.sh, valid, a.D, half);
+  if (cur >= 0) {
+    ksrc.issue(kt_at, cur);
+    vsrc.issue(vt_at, cur);
+    kmask = key_mask(cur);
   }
+  const float iq = qr.inv_norm(a.eps);
   const float thq = hp.thr / iq;  // s > thr  <=>  (k . q)/|k| > thr |q|
+  const float riq = hp.r * iq;
   f32x16 o[NDH];
 #pragma unroll
   for (int dblk = 0; dblk < NDH; ++dblk)
@@ -910,105 +888,70 @@ void fwd_live_kernel(FwdKArgs a) {
 
   while (cur >= 0) {
     const int k0 = cur * kUnit;
+    wait_vmcnt<0>();  // the unit's rows have landed
     // S^T = K Q^T on the raw rows (exact products of the inputs, fp32
-    // accumulation), scaled by 1/|k_j| in fp32 below: register r -> key
-    // k0 + rowof(r, half), lane -> query i
-    vzero(kc);
-    f32x16 s;
-    float s2k = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+    // accumulation): register r -> key k0 + rowof(r, half), lane -> query i
+    f32x16 s, slo;  // fp32: s + slo
+    frag va[NDH * NC];
+    float ik, iv;  // 1/|k|, 1/|v| of the lane's key row m
     {
-      frag qf[NKS];
+      float s2k, s2v;
+      {
+        frag kf[NKS];
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) qf[ks] = qsh[ks][lane];
-      if constexpr (sizeof(T) == 2) {
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-          s = M::mma_ng(kc[ks], qf[ks], s);
-          s2k = frag_dot(kc[ks], kc[ks], s2k);
-        }
-        guard_frags(kc);
-        guard_frags(qf);
-      } else {
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-          s = M::mma(kc[ks], qf[ks], s);
-          s2k = frag_dot(kc[ks], kc[ks], s2k);
-        }
+        for (int ks = 0; ks < NKS; ++ks) kf[ks] = U::row_frag(kt, rb, ks);
+        vzero(kf);
+        s = unit_product<T>(kf, qr.f, &slo);
+        s2k = row_dot<T>(kf, kf);
+        guard_run(kf, s);
       }
+      {
+        frag vf[NKS];
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) vf[ks] = U::row_frag(vt, rb, ks);
+        vzero(vf);
+        s2v = row_dot<T>(vf, vf);
+      }
+#pragma unroll
+      for (int dblk = 0; dblk < NDH; ++dblk)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) va[dblk * NC + c] = U::col_frag(vt, cb, dblk, c);
+      ik = k0 + m < a.Tk && kmask == 0u ? inv_len_of<T>(half_sum(s2k), a.eps) : 0.0f;
+      iv = inv_len_of<T>(half_sum(s2v), a.eps);
     }
-    // each operand's registers take the next unit's rows as soon as they are
-    // free, so those loads run behind the rest of this unit's work (past the
-    // last unit, the current one again, a cache hit: every iteration then
-    // waits for the same count)
+    // every read of the staged rows has returned: the next unit's copies run
+    // behind the rest of this unit's work
     int nxt = -1;  // this wave's next unit: S positions on in the row's walk
     for (int w = 0; w < S; ++w) {
       nxt = walk.next();
       if (nxt < 0) break;
     }
-    const int nl = nxt >= 0 ? nxt : cur;
-    const bool kok_c = kok;
-    load_k(nl, kc);
-    kok = key_ok(nl);
-    // 1/|k_j| and 1/|v_j| of the lane's key row, to LDS (read back in
-    // register order), then V^T by identity MFMA
-    vzero(vc);
-    float ivl;  // this lane's 1/|v| (its row m)
-    {
-      float s2v = 0.0f;
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) s2v = frag_dot(vc[ks], vc[ks], s2v);
-      s2v = half_sum(s2v);
-      s2k = half_sum(s2k);
-      const float iv = inv_len(s2v, a.eps);
-      ivl = iv;
-      const float ik = kok_c ? inv_len(s2k, a.eps) : 0.0f;
-      wave_lds_sync();
-      if (half == 0) {
-        sv[m] = iv;
-        sk[m] = ik;
-      }
-      unit_mask_table<false>(mt, nullptr, qu * kUnit - k0 - 31, hp, lane);
-      wave_lds_sync();
+    wave_lds_sync();
+    if (nxt >= 0) {
+      ksrc.issue(kt_at, nxt);
+      vsrc.issue(vt_at, nxt);
+      kmask = key_mask(nxt);
     }
+    // 1/|k_j| and 1/|v_j| to LDS, read back in register order
+    if (half == 0) {
+      sk[m] = ik;
+      if constexpr (kPow2Rows<T>) {
+        const Pow2Split p(iv);
+        sv[m] = p.w;
+        sc_w[wave][0][m] = (f16)p.c1;
+        sc_w[wave][1][m] = (f16)p.c2;
+      } else {
+        sv[m] = iv;
+      }
+    }
+    unit_mask_table<false>(mt, nullptr, qu * kUnit - k0 - 31, hp, lane);
+    wave_lds_sync();
     {
       float ksc[16];
       read_row_scales(sk, half, ksc);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] *= ksc[r];
+      for (int r = 0; r < 16; ++r) scale_pair<T>(s, slo, r, ksc[r]);
     }
-    frag ta[NDH * NC];
-    frag id[NC];  // formed per unit: fewer registers held across the loop
-#pragma unroll
-    for (int c = 0; c < NC; ++c) id[c] = ident_frag<T>(c, lane);
-    // fp16: each lane's V row takes its 1/|v| before the transposes (in fp32,
-    // rounded once to fp16: the value the transposed row would get), which
-    // holds one scale per lane instead of sixteen.  The scheduling barriers
-    // keep the conversions in place: hoisted next to the S products they
-    // held 32 more values at once and spilled 9 VGPRs (live 42 -> 32 us at
-    // configs[1] in fp16 without the spill)
-    if constexpr (kScaleRowsNotWeights<T>) {
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < NKS; ++ks)
-#pragma unroll
-        for (int e = 0; e < PER; ++e) vc[ks][e] = (T)((float)vc[ks][e] * ivl);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int dblk = 0; dblk < NDH; ++dblk) {
-      f32x16 tr;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) tr[r] = 0.0f;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) tr = M::mma_ng(vc[dblk * NC + c], id[c], tr);
-#pragma unroll
-      for (int c = 0; c < NC; ++c) ta[dblk * NC + c] = M::pack(tr, c * PER);
-    }
-    guard_frags(vc);
-    guard_frags(id);
-    load_v(nl, vc);
     // P^T[j][i] = alpha_ij m_ij / |v_j|: every lane forms its pair's weight
     // branch-free (alpha = 0 below the threshold, the mask, 0 outside the
     // window, from the unit's table: register r holds distance i - k0 - 8half
@@ -1020,7 +963,7 @@ void fwd_live_kernel(FwdKArgs a) {
       const float* mrow = mt + (l32 - 8 * half + 8);  // entry 23 - (16(r/8) + r%8): a constant offset
       auto body = [&](int r) {
         const int off = 16 * (r >> 3) + (r & 7);
-        const float av = fmaxf(trim(s[r] * iq, hp.r), 0.0f);
+        const float av = pair_root<T>(s[r], slo[r], iq, riq, hp.r);
         float p = av * av * mrow[23 - off];
         if (a.drop.on) p *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
         s[r] = p;
@@ -1035,12 +978,21 @@ void fwd_live_kernel(FwdKArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) body(r);
       }
-      if constexpr (!kScaleRowsNotWeights<T>) {
-        float vsc[16];
-        read_row_scales(sv, half, vsc);
+      float vsc[16];
+      read_row_scales(sv, half, vsc);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] *= vsc[r];
-      }
+      for (int r = 0; r < 16; ++r) s[r] *= vsc[r];
+    }
+    if constexpr (kPow2Rows<T>) {
+      // c2 differs from 1 only for rows shorter than 2^-15
+      const bool tiny = __ballot(iv > 32768.0f) != 0ull;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int dblk = 0; dblk < NDH; ++dblk) {
+          scale_slots(va[dblk * NC + c], sc_w[wave][0], c, half);
+          if (tiny) scale_slots(va[dblk * NC + c], sc_w[wave][1], c, half);
+        }
     }
     // H^T[d][i] += sum_j V^T[d][j] P^T[j][i]
     frag pb[NC];
@@ -1049,17 +1001,16 @@ void fwd_live_kernel(FwdKArgs a) {
 #pragma unroll
     for (int c = 0; c < NC; ++c)
 #pragma unroll
-      for (int dblk = 0; dblk < NDH; ++dblk) o[dblk] = M::mma_ng(ta[dblk * NC + c], pb[c], o[dblk]);
-    guard_frags(ta);
-    guard_frags(pb);
-    if (nxt < 0) break;
+      for (int dblk = 0; dblk < NDH; ++dblk) o[dblk] = M::mma_ng(va[dblk * NC + c], pb[c], o[dblk]);
+    guard_run(va, o[NDH - 1]);
+    guard_keep(pb);
     cur = nxt;
   }
 
   if constexpr (S > 1) {
-    // waves 1..S-1 hand their H^T to wave 0 (each in its own wbuf row),
+    // waves 1..S-1 hand their H^T to wave 0 (each in its own stage row),
     // which adds them in wave order
-    auto part = [&](int w) { return reinterpret_cast<float(*)[kWave]>(wbuf[w]); };
+    auto part = [&](int w) { return reinterpret_cast<float(*)[kWave]>(stage[w]); };
     if (wave > 0)
 #pragma unroll
       for (int dblk = 0; dblk < NDH; ++dblk)
@@ -1072,6 +1023,12 @@ void fwd_live_kernel(FwdKArgs a) {
       for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[dblk][r] += part(w)[dblk * 16 + r][lane];
+  }
+  // D = 16: the block's rows past D hold the repeated columns' products
+  if constexpr (DP == 32) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (KS * creg_ks<T>(0, r) >= a.D) o[0][r] = 0.0f;
   }
   // TanhNorm per query row (lane -> query, registers -> d), y in (B,T,H,D)
   float ss = 0.0f;
@@ -1092,10 +1049,6 @@ void fwd_live_kernel(FwdKArgs a) {
 static int64_t khat_bytes(const Geometry& g) {
   return round_up((int64_t)g.B * g.H * g.Tk_pad * g.DP * (int64_t)sizeof(ScreenOp), 256);  // fp16 rows
 }
-// Rows (32-query units) below which the live pass splits each row's units
-// over several waves: about two waves per SIMD of the chip.
-constexpr int64_t kLiveSplitWaves = 2048;
-
 // Workspace: [K^][screen plan table]
 size_t fwd_ws_bytes(const Geometry& g) { return khat_bytes(g) + screen_plan_bytes(g); }
 
@@ -1140,19 +1093,15 @@ static hipError_t launch_fwd_t(const FwdCall& c) {
   // A launch with few rows (under about two waves per SIMD) splits each
   // row's live units over S waves (DP <= 64: the S waves' LDS fits)
   const int64_t rows = (int64_t)2 * g.nqt * g.B * g.H;
-  const int S = DP > 64 ? 1 : (rows * 4 <= kLiveSplitWaves ? 4 : (rows * 2 <= kLiveSplitWaves ? 2 : 1));
+  const int S = split_waves<T>(rows);
   const dim3 grid((unsigned)(2 * g.nqt), (unsigned)(g.B * g.H));
   timer_begin(3, c.stream);
-  if constexpr (DP <= 64) {
-    if (S == 4)
-      hipLaunchKernelGGL((fwd_live_kernel<T, DP, 4>), grid, dim3(256), 0, c.stream, fa);
-    else if (S == 2)
-      hipLaunchKernelGGL((fwd_live_kernel<T, DP, 2>), grid, dim3(128), 0, c.stream, fa);
-    else
-      hipLaunchKernelGGL((fwd_live_kernel<T, DP, 1>), grid, dim3(64), 0, c.stream, fa);
-  } else {
+  if (S == 4)
+    hipLaunchKernelGGL((fwd_live_kernel<T, DP, 4>), grid, dim3(256), 0, c.stream, fa);
+  else if (S == 2)
+    hipLaunchKernelGGL((fwd_live_kernel<T, DP, 2>), grid, dim3(128), 0, c.stream, fa);
+  else
     hipLaunchKernelGGL((fwd_live_kernel<T, DP, 1>), grid, dim3(64), 0, c.stream, fa);
-  }
   timer_end(3, c.stream);
   return hipGetLastError();
 }

@@ -104,6 +104,15 @@ int decode_chunk_keys();
 int decode_max_chunks(int max_len);
 hipError_t launch_decode(const DecodeCall& c);
 
+// Waves that share a row (32-query or 32-key unit) in the live, dq and dK/dV
+// passes: launches with few rows split each row's units, up to about two
+// waves per SIMD of the chip (2-byte types) or four (fp32).
+template <typename T>
+inline int split_waves(int64_t rows) {
+  const int64_t most = sizeof(T) == 2 ? 2048 : 4096;
+  return rows * 4 <= most ? 4 : (rows * 2 <= most ? 2 : 1);
+}
+
 // Optional event pairs around one kernel's launches (msa_timer_arm).
 void timer_begin(int kernel, hipStream_t s);
 void timer_end(int kernel, hipStream_t s);
