@@ -176,7 +176,7 @@ __device__ inline void write_norm_bwd(const f32x16 (&acc)[DP / 32], const typena
 template <typename T, int DP>
 constexpr int dq_waves() { return sizeof(T) * DP <= 64 ? 3 : (sizeof(T) * DP <= 128 ? 2 : 1); }
 
-template <typename T, int DP, int S>
+template <typename T, int DP, int S, bool DROP>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(dq_waves<T, DP>())))
 void dq_kernel(BwdKArgs a) {
   using M = Mma<T>;
@@ -390,13 +390,13 @@ void dq_kernel(BwdKArgs a) {
         const int off = 16 * (r >> 3) + (r & 7);
         const float av = pair_root<T>(s[r], slo[r], iql, riq, hp.r);
         float u = av * dp[r];
-        if (a.drop.on) u *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
+        if constexpr (DROP) u *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
         const float um = u * mrow[23 - off];
         dr_acc = fmaf(um, 1.0f - av, dr_acc);
         dw_acc = fmaf(u * av, mrow[64 + 23 - off], dw_acc);
         dp[r] = um;
       };
-      if (a.drop.on) {  // the pair's hash only where some lane may pass
+      if constexpr (DROP) {  // the pair's hash only where some lane may pass
         const uint32_t pm0 = pass_mask(s, thq);
         for_each_set(pm0, body);
 #pragma unroll
@@ -404,12 +404,10 @@ void dq_kernel(BwdKArgs a) {
           if (((pm0 >> r) & 1u) == 0u) dp[r] = 0.0f;
       } else {  // every register: a = 0 gives no term, and no mask or branches
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          body(r);
-          if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four registers' terms live at a time
-        }
+        for (int r = 0; r < 16; ++r) body(r);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
     // dq^T[d][i] += sum_j K^T[d][j] (ds/|k|)^T[j][i] (fp16: 1/|k|'s power of
     // two goes to the K columns, the rest to ds)
     {
@@ -494,7 +492,7 @@ constexpr int dkdv_waves() { return sizeof(T) * DP <= 128 ? 2 : 1; }
 template <typename T>
 constexpr bool kLateColumns = sizeof(T) == 4;
 
-template <typename T, int DP, int S>
+template <typename T, int DP, int S, bool DROP>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(dkdv_waves<T, DP>())))
 void dkdv_kernel(BwdKArgs a) {
   using M = Mma<T>;
@@ -584,7 +582,7 @@ void dkdv_kernel(BwdKArgs a) {
   const typename U::Source qsrc((const T*)a.q + b * a.qs.sb + h * a.qs.sh, a.qs.st, a.Tq, a.D, lane);
   const typename U::Source hsrc((const T*)a.dh + (int64_t)bh * a.Tq_pad * DP, DP, (int)a.Tq_pad, DP, lane);
   const float* iq0 = a.iqs + (int64_t)bh * a.Tq_pad;
-  const uint32_t rb = U::row_base(lane), cb = U::col_base(lane);
+  uint32_t rb = U::row_base(lane), cb = U::col_base(lane);
   // D = 16: the staged columns past D repeat the first ones (dh rows hold DP)
   auto zero_tail = [&](frag (&f)[NKS]) {
     if constexpr (DP == 32) {
@@ -615,6 +613,10 @@ void dkdv_kernel(BwdKArgs a) {
 
   while (cur >= 0) {
     const int q0 = cur * kUnit;
+    if constexpr (!__is_same(T, bf16)) {
+      rederive(rb);
+      rederive(cb);
+    }
     wait_vmcnt<0>();  // the unit's rows have landed
     const float iqc = iqv;
     if (half == 0) {
@@ -684,6 +686,7 @@ void dkdv_kernel(BwdKArgs a) {
       scale_pair<T>(s, slo, r, qsc[r]);
       if constexpr (kPow2Rows<T>) dp[r] *= ivl;
     }
+    __builtin_amdgcn_sched_barrier(0);
     // every lane forms its pair's weight and ds branch-free (the mask, 0
     // outside the window, from the unit's table: entry 16(r/8) + r%8 + 8half
     // - l32 + 31 for register r), for every register; with dropout, only for
@@ -695,12 +698,12 @@ void dkdv_kernel(BwdKArgs a) {
         const int off = 16 * (r >> 3) + (r & 7);
         const float av = pair_root<T>(s[r], slo[r], ikl, rik, hp.r);
         float mk = mrow[off];
-        if (a.drop.on) mk *= dropout_factor(a.drop, bh, q0 + 8 * half + off, j);
+        if constexpr (DROP) mk *= dropout_factor(a.drop, bh, q0 + 8 * half + off, j);
         const float am = av * mk;
         s[r] = av * am;
         dp[r] = am * dp[r];
       };
-      if (a.drop.on) {  // the pair's hash only where some lane may pass
+      if constexpr (DROP) {  // the pair's hash only where some lane may pass
         const uint32_t pm0 = pass_mask(s, thk);
         for_each_set(pm0, body);
 #pragma unroll
@@ -711,6 +714,7 @@ void dkdv_kernel(BwdKArgs a) {
         for (int r = 0; r < 16; ++r) body(r);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
     // ds/|q| (fp16: 1/|q|'s power of two goes to the Q columns, the rest here)
     if constexpr (kPow2Rows<T>) read_row_scales(sw_w[wave], half, qsc);
 #pragma unroll
@@ -827,22 +831,29 @@ static hipError_t launch_bwd_t(const BwdCall& c) {
     const int64_t rows = (int64_t)2 * tiles * g.B * g.H;
     return split_waves<T>(rows);
   };
+  auto launch_split = [&](int S, auto&& fn) {
+    auto with = [&](auto drop) {
+      if (S == 4) fn(std::integral_constant<int, 4>{}, drop);
+      else if (S == 2) fn(std::integral_constant<int, 2>{}, drop);
+      else fn(std::integral_constant<int, 1>{}, drop);
+    };
+    if (c.drop.on) with(std::true_type{});
+    else with(std::false_type{});
+  };
   const dim3 qgrid((unsigned)(2 * g.nqt), (unsigned)(g.B * g.H)), kgrid((unsigned)(2 * g.nkt), (unsigned)(g.B * g.H));
   timer_begin(5, c.stream);
-  switch (split(g.nqt)) {
-    case 4: hipLaunchKernelGGL((dq_kernel<T, DP, 4>), qgrid, dim3(256), 0, c.stream, ka); break;
-    case 2: hipLaunchKernelGGL((dq_kernel<T, DP, 2>), qgrid, dim3(128), 0, c.stream, ka); break;
-    default: hipLaunchKernelGGL((dq_kernel<T, DP, 1>), qgrid, dim3(64), 0, c.stream, ka);
-  }
+  launch_split(split(g.nqt), [&](auto waves, auto drop) {
+    constexpr int S = decltype(waves)::value;
+    hipLaunchKernelGGL((dq_kernel<T, DP, S, decltype(drop)::value>), qgrid, dim3(64 * S), 0, c.stream, ka);
+  });
   timer_end(5, c.stream);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   timer_begin(4, c.stream);
-  switch (split(g.nkt)) {
-    case 4: hipLaunchKernelGGL((dkdv_kernel<T, DP, 4>), kgrid, dim3(256), 0, c.stream, ka); break;
-    case 2: hipLaunchKernelGGL((dkdv_kernel<T, DP, 2>), kgrid, dim3(128), 0, c.stream, ka); break;
-    default: hipLaunchKernelGGL((dkdv_kernel<T, DP, 1>), kgrid, dim3(64), 0, c.stream, ka);
-  }
+  launch_split(split(g.nkt), [&](auto waves, auto drop) {
+    constexpr int S = decltype(waves)::value;
+    hipLaunchKernelGGL((dkdv_kernel<T, DP, S, decltype(drop)::value>), kgrid, dim3(64 * S), 0, c.stream, ka);
+  });
   timer_end(4, c.stream);
   return hipGetLastError();
 }

@@ -688,6 +688,11 @@ __device__ constexpr int lds_swz(int R) {
   else return b1 | (b3 << 1) | ((b0 ^ b2) << 2) | (b0 << 3);
 }
 
+// Keeps the compiler from holding values derived from x across loop iterations
+// (a few instructions each time instead of a register each; a spilled register
+// would be reloaded behind the copies in flight, and wait for them).
+__device__ inline void rederive(uint32_t& x) { asm volatile("" : "+v"(x)); }
+
 // ---------------------------------------------------------------------------
 // A 32-row unit of a (B,T,H,D) tensor staged in a wave's own LDS.  The rows
 // come by direct DMA, each instruction moving whole rows (1 KiB: 8 rows of
@@ -724,24 +729,28 @@ struct UnitTile {
     const char* base;  // row 0 of the head
     uint32_t stb;
     int rows;          // rows of the tensor (rows past them read the last one)
-    uint32_t lrow, cb;
+    uint32_t off, cb;  // the lane's row of an instruction and its 16-byte chunk, in bytes
     uint32_t cmask;    // D = 16 of DP = 32: chunks past D re-read the row's first ones
     __device__ Source(const T* head, int64_t st, int rows_, int D, int lane)
         : base((const char*)head), stb((uint32_t)(st * (int64_t)sizeof(T))), rows(rows_),
-          lrow((uint32_t)(lane / CPR)), cb((uint32_t)((lane % CPR) ^ swz(lane / CPR)) << 4),
+          off((uint32_t)(lane / CPR) * stb), cb((uint32_t)((lane % CPR) ^ swz(lane / CPR)) << 4),
           cmask(DP == 32 && D < DP ? (uint32_t)(D * (int)sizeof(T) - 1) : 0xffffffffu) {}
     // Starts the copy of unit u to LDS address `lds` (wave-uniform; RPI rows, 1 KiB, an
     // instruction).  Row offsets stay below 2^32 bytes: 64 rows span less.
-    __device__ inline void issue(LdsChar* lds, int u) const {
+    template <typename P>
+    __device__ inline void issue(P lds, int u) const {
       const char* ub = base + (int64_t)u * kUnit * stb;
       const int last = rows - 1 - u * kUnit;
       if (last >= kUnit - 1) {
+        uint32_t o = off;
+        rederive(o);
 #pragma unroll
-        for (int i = 0; i < NI; ++i) dma(ub + (int64_t)(i * RPI) * stb + (uint32_t)(lrow * stb + chunk(i)), lds, i);
+        for (int i = 0; i < NI; ++i) dma(ub + (int64_t)(i * RPI) * stb + (uint32_t)(o + chunk(i)), lds, i);
       } else {
+        const int lrow = (int)(threadIdx.x & 63) / CPR;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
-          const int r = i * RPI + (int)lrow;
+          const int r = i * RPI + lrow;
           dma(ub + (uint32_t)((uint32_t)(r < last ? r : last) * stb + chunk(i)), lds, i);
         }
       }
@@ -750,7 +759,8 @@ struct UnitTile {
       const uint32_t c = cb ^ (uint32_t)(swz((i * RPI) & 15) << 4);
       return DP == 32 ? c & cmask : c;
     }
-    __device__ static inline void dma(const char* src, LdsChar* lds, int i) {
+    template <typename P>
+    __device__ static inline void dma(const char* src, P lds, int i) {
       __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
                                        (void __attribute__((address_space(3)))*)(lds + i * 1024), 16, 0, 0);
     }
@@ -802,6 +812,76 @@ struct UnitTile {
       }
       return v;
     }
+  }
+};
+
+// All of a 2-byte unit's column fragments (UnitTile::col_frag), as one block of
+// reads with its wait: the transposing builtin makes the compiler wait for
+// every copy in flight first, and in the group form the next tile's copies are.
+// `at` is the LDS address of the unit's rows plus col_base.
+template <typename T, int DP>
+__device__ inline void col_frags_now(typename Mma<T>::frag (&f)[DP / 16], uint32_t at) {
+  using U = UnitTile<T, DP>;
+  typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
+  typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4;
+  constexpr int R4 = 4 * U::ROWB, R16 = 16 * U::ROWB;
+  constexpr uint32_t kJ = (uint32_t)(U::swz(4) << 4);  // rows + 4
+  auto join = [](i32x2 a, i32x2 b) { return __builtin_bit_cast(typename Mma<T>::frag, i32x4{a[0], a[1], b[0], b[1]}); };
+  if constexpr (DP == 32) {
+    i32x2 x[4];
+    asm volatile("ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %5 offset:%6\n\t"
+                 "ds_read_b64_tr_b16 %2, %4 offset:%7\n\tds_read_b64_tr_b16 %3, %5 offset:%8\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
+                 : "v"(at), "v"(at ^ kJ), "n"(R4), "n"(R16), "n"(R16 + R4));
+    f[0] = join(x[0], x[1]);
+    f[1] = join(x[2], x[3]);
+  } else {
+#pragma unroll
+    for (int d = 0; d < DP / 32; d += 2) {  // column blocks d, d + 1: chunks 4 apart, as rows 4 apart
+      const uint32_t a0 = at ^ (uint32_t)(4 * d << 4), a1 = a0 ^ kJ;
+      static_assert(kJ == 4 << 4, "rows + 4 and the next column block swizzle alike");
+      i32x2 x[8];
+      asm volatile("ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %9 offset:%10\n\t"
+                   "ds_read_b64_tr_b16 %2, %8 offset:%11\n\tds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
+                   "ds_read_b64_tr_b16 %4, %9\n\tds_read_b64_tr_b16 %5, %8 offset:%10\n\t"
+                   "ds_read_b64_tr_b16 %6, %9 offset:%11\n\tds_read_b64_tr_b16 %7, %8 offset:%12\n\t"
+                   "s_waitcnt lgkmcnt(0)"
+                   : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
+                   : "v"(a0), "v"(a1), "n"(R4), "n"(R16), "n"(R16 + R4));
+      f[2 * d] = join(x[0], x[1]);
+      f[2 * d + 1] = join(x[2], x[3]);
+      f[2 * d + 2] = join(x[4], x[5]);
+      f[2 * d + 3] = join(x[6], x[7]);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Group form of a pass: the four waves of a 256-thread block hold four
+// adjacent units of one head (128 rows) and walk the other side's 64-row tiles
+// together.  A tile of two tensors X, Y (K, V or Q, dh) is staged once for the
+// block, wave w copying one of its four units; what depends on the other side
+// alone (1/|x|, the mask table of the block's 191 distances) is formed once by
+// the 256 threads.  Three tiles are in LDS: step n computes tile n while tile
+// n+1 has its factors formed and tile n+2 is copied, with one barrier a step.
+// ---------------------------------------------------------------------------
+constexpr int kGroup = 4;  // units (waves) of a block
+template <typename T, int DP>
+struct GroupStage {
+  using U = UnitTile<T, DP>;
+  static constexpr int TILEB = 4 * U::BYTES;  // X unit 0, X unit 1, Y unit 0, Y unit 1
+  static constexpr int NB = 3;
+  // 1/max(|x|, eps) of the staged tile's rows: two threads a row, X rows first
+  // (row t/2 of 128), every lane of the pair getting the value.
+  __device__ static inline float row_factor(const char* tile, int t, float eps) {
+    constexpr int CH = U::CPR / 2;  // 16-byte chunks per thread
+    const int row = t >> 1, r32 = row & 31;
+    const char* p = tile + (row >> 5) * U::BYTES + r32 * U::ROWB;
+    typename U::frag f[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+      f[c] = *reinterpret_cast<const typename U::frag*>(p + ((((t & 1) * CH + c) ^ U::swz(r32)) << 4));
+    return inv_len_of<T>(group_sum<2>(row_dot<T>(f, f)), eps);
   }
 };
 

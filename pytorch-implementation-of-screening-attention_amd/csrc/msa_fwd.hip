@@ -785,7 +785,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // wave 0 through LDS, which adds them in wave order (fixed, so results repeat
 // bitwise) and runs the epilogue.
 // ---------------------------------------------------------------------------
-template <typename T, int DP, int S>
+template <typename T, int DP, int S, bool DROP>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(unit_waves<T, DP>())))
 void fwd_live_kernel(FwdKArgs a) {
   using M = Mma<T>;
@@ -852,7 +852,7 @@ void fwd_live_kernel(FwdKArgs a) {
   const int m = perm_row(l32);
   const typename U::Source ksrc((const T*)a.k + b * a.ks.sb + h * a.ks.sh, a.ks.st, a.Tk, a.D, lane);
   const typename U::Source vsrc((const T*)a.v + b * a.vs.sb + h * a.vs.sh, a.vs.st, a.Tk, a.D, lane);
-  const uint32_t rb = U::row_base(lane), cb = U::col_base(lane);
+  uint32_t rb = U::row_base(lane), cb = U::col_base(lane);
   // 1/|k| is 0 for keys past Tk and for masked keys, so they never pass the
   // threshold and their P is exactly 0
   auto key_mask = [&](int u) -> unsigned {  // the mask byte, tested when the unit is computed
@@ -888,6 +888,10 @@ void fwd_live_kernel(FwdKArgs a) {
 
   while (cur >= 0) {
     const int k0 = cur * kUnit;
+    if constexpr (!__is_same(T, bf16)) {
+      rederive(rb);
+      rederive(cb);
+    }
     wait_vmcnt<0>();  // the unit's rows have landed
     // S^T = K Q^T on the raw rows (exact products of the inputs, fp32
     // accumulation): register r -> key k0 + rowof(r, half), lane -> query i
@@ -905,6 +909,7 @@ void fwd_live_kernel(FwdKArgs a) {
         s2k = row_dot<T>(kf, kf);
         guard_run(kf, s);
       }
+      __builtin_amdgcn_sched_barrier(0);
       {
         frag vf[NKS];
 #pragma unroll
@@ -951,6 +956,7 @@ void fwd_live_kernel(FwdKArgs a) {
       read_row_scales(sk, half, ksc);
 #pragma unroll
       for (int r = 0; r < 16; ++r) scale_pair<T>(s, slo, r, ksc[r]);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // P^T[j][i] = alpha_ij m_ij / |v_j|: every lane forms its pair's weight
     // branch-free (alpha = 0 below the threshold, the mask, 0 outside the
@@ -965,10 +971,10 @@ void fwd_live_kernel(FwdKArgs a) {
         const int off = 16 * (r >> 3) + (r & 7);
         const float av = pair_root<T>(s[r], slo[r], iq, riq, hp.r);
         float p = av * av * mrow[23 - off];
-        if (a.drop.on) p *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
+        if constexpr (DROP) p *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
         s[r] = p;
       };
-      if (a.drop.on) {
+      if constexpr (DROP) {
         const uint32_t pm0 = pass_mask(s, thq);
         for_each_set(pm0, body);
 #pragma unroll
@@ -978,6 +984,7 @@ void fwd_live_kernel(FwdKArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) body(r);
       }
+      __builtin_amdgcn_sched_barrier(0);
       float vsc[16];
       read_row_scales(sv, half, vsc);
 #pragma unroll
@@ -1096,12 +1103,17 @@ static hipError_t launch_fwd_t(const FwdCall& c) {
   const int S = split_waves<T>(rows);
   const dim3 grid((unsigned)(2 * g.nqt), (unsigned)(g.B * g.H));
   timer_begin(3, c.stream);
-  if (S == 4)
-    hipLaunchKernelGGL((fwd_live_kernel<T, DP, 4>), grid, dim3(256), 0, c.stream, fa);
-  else if (S == 2)
-    hipLaunchKernelGGL((fwd_live_kernel<T, DP, 2>), grid, dim3(128), 0, c.stream, fa);
-  else
-    hipLaunchKernelGGL((fwd_live_kernel<T, DP, 1>), grid, dim3(64), 0, c.stream, fa);
+  auto launch = [&](auto drop) {
+    constexpr bool DROP = decltype(drop)::value;
+    if (S == 4)
+      hipLaunchKernelGGL((fwd_live_kernel<T, DP, 4, DROP>), grid, dim3(256), 0, c.stream, fa);
+    else if (S == 2)
+      hipLaunchKernelGGL((fwd_live_kernel<T, DP, 2, DROP>), grid, dim3(128), 0, c.stream, fa);
+    else
+      hipLaunchKernelGGL((fwd_live_kernel<T, DP, 1, DROP>), grid, dim3(64), 0, c.stream, fa);
+  };
+  if (c.drop.on) launch(std::true_type{});
+  else launch(std::false_type{});
   timer_end(3, c.stream);
   return hipGetLastError();
 }
