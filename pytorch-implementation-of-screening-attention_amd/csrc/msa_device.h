@@ -123,6 +123,23 @@ template <> struct Mma<bf16> {
   }
 };
 
+// int8 (the screen only): 32x32x32, int32 accumulation; a lane's 16 slots are
+// 16 bytes of its row.
+typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4;
+typedef __attribute__((__vector_size__(16 * sizeof(int)))) int i32x16;
+template <> struct Mma<int8_t> {
+  static constexpr int KS = 32;
+  static constexpr int PER = 16;
+  typedef i32x4 frag;
+  typedef i32x16 acc;
+  typedef int acc_elem;
+  __device__ static inline i32x16 mma_ng(frag a, frag b, i32x16 c) {
+    return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
+  }
+  __device__ static inline frag load(const int8_t* p) { return *reinterpret_cast<const frag*>(p); }
+  __device__ static inline int max(int x, int y) { return x > y ? x : y; }
+};
+
 // fp16: the same 32x32x16 operand layout and pass count as bf16
 // (v_mfma_f32_32x32x16_f16), so every layout map and the source-operand guard
 // apply unchanged.
@@ -130,6 +147,9 @@ template <> struct Mma<f16> {
   static constexpr int KS = 16;
   static constexpr int PER = 8;
   typedef f16x8 frag;
+  typedef f32x16 acc;
+  typedef float acc_elem;
+  __device__ static inline float max(float x, float y) { return fmaxf(x, y); }
   __device__ static inline f32x16 mma_ng(frag a, frag b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }

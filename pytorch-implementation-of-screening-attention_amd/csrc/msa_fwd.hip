@@ -54,6 +54,7 @@ namespace msa {
 // are ORed).
 // ---------------------------------------------------------------------------
 constexpr int kScreenBlocksPerLane = 256;
+constexpr int kScreenMaxSeg = 256;  // steps of an item at most
 struct ScreenItem {
   int bh, grp, lo, hi;  // head, 4-query-tile group, tile offsets qt - kt in [lo, hi]
   float r, w;           // the head's r_h, w_h (copied, so one load gives the screen all)
@@ -300,7 +301,8 @@ size_t screen_plan_bytes(const Geometry& g) {
 }
 
 // ---------------------------------------------------------------------------
-// Screen operands.  Every input type screens on fp16 MFMA operands: K^ =
+// Screen operands.  Every input type screens on fp16 MFMA operands (long
+// windows of 2-byte inputs on int8 ones, below): K^ =
 // k/|k| rounded to fp16, and each raw query row rounded to fp16, so each vote
 // sees s up to their rounding: |s_screen - s| <= (u_k + u_q + u_k u_q)
 // sum_d |q^_d k^_d| <= u_k + u_q + u_k u_q (unit roundoffs, unit vectors).
@@ -324,8 +326,23 @@ size_t screen_plan_bytes(const Geometry& g) {
 // rounding above, fp32 accumulation of D <= 128 products ((D+3) 2^-24) and
 // the fp32 1/|q| and 1/|k|.
 // ---------------------------------------------------------------------------
-using ScreenOp = f16;              // the screen's MFMA operand type
-constexpr float kKhatScale = 1024.0f;  // K^ is stored times 2^10
+//   int8: heads of long windows (int8_window) of a launch for which
+//     screens_int8 holds, at twice the MFMA rate on half the K^ bytes.  Row x of q is round(x g_q), g_q =
+//     127/max|x|; k^ = k/|k| is round(k^ g_k), g_k common to the 32 keys of a
+//     unit (127 over the unit's largest component), so acc = Q K is exact in
+//     int32 and comparable within a unit.  What the rounding took is measured,
+//     not bounded a priori: e_q and e_k are the lengths of the rounding errors
+//     of q^ and k^ (e_k the unit's largest), and
+//       |s - acc/(g_q g_k |q|)| <= e_q |k^| + (1 + e_q) e_k <= e_q + (1 + e_q) e_k.
+//     A unit is marked iff acc > g_k (A - B e_k) for some pair, with N = g_q |q|,
+//     A = (1 - 1/r - 2e-5 - e_q) N and B = (1 + e_q) N.  At D = 64 and normal
+//     rows e_q + e_k is about 0.014, which marks about 1.6 times the units that
+//     hold a live pair; the live pass takes the others' bits back.  A bound by
+//     lengths is loose for single pairs, but the only one that never misses.
+//     B=1 T=100,000 bf16 at initialisation, windows 512 .. 100,000: screen
+//     2620 -> 1681 us, live pass 425 -> 706 (its DMA of the dead units' rows).
+constexpr float kKhatScale = 1024.0f;  // fp16 K^ is stored times 2^10
+constexpr float kInt8Slack = 2e-5f;    // fp32 rounding of s, |q|, |k|, e_q and e_k
 template <typename T>
 constexpr float kScreenSlack = sizeof(T) == 2 ? 4.8828125e-4f + 1e-5f    // 2^-11 + 1e-5
                                               : 9.765625e-4f + 1e-5f;    // 2^-10 + 1e-5
@@ -376,10 +393,36 @@ __device__ inline float row_pow2(float mx) {
   return ldexpf(1.0f, e);
 }
 
+// int8 of y (|y| <= 127, in its low byte) and the rounding's error y - round(y).
+__device__ inline uint32_t round_int8(float y, float& err) {
+  const float f = y + 12582912.0f;  // 1.5 * 2^23: the sum's low bits are round(y)
+  err = y - (f - 12582912.0f);
+  return (uint32_t)__float_as_int(f);
+}
+__device__ inline uint32_t pack4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {  // low bytes, a lowest
+  return __builtin_amdgcn_perm(__builtin_amdgcn_perm(d, c, 0x0c0c0400u), __builtin_amdgcn_perm(b, a, 0x0c0c0400u),
+                               0x05040100u);
+}
+
+// Heads that screen on int8 operands, where the launch takes them
+// (screens_int8): windows of at least 4096 positions.  Shorter ones don't pay
+// for the heavier row preparation and the live pass's walk over units that
+// turn out dead: us a call, fp16 -> int8 for all heads: causal bf16 step at
+// initialisation, windows T/16 .. T, T = 4096 186 -> 189, T = 8192 208 -> 195
+// (D = 128: 315 -> 261); forward T = 30000 322 -> 262, with windows of
+// 32 .. 512 49 -> 57.
+constexpr int kInt8Window = 4096;
+__device__ inline bool int8_window(float w, int Tq, int Tk) {
+  return w >= (float)kInt8Window && (Tq > Tk ? Tq : Tk) >= kInt8Window;
+}
+
+// Scale and error of a key unit's int8 rows.
+struct KeyUnitScale { float g, e; };  // g_k, e_k
+
 // 16-byte chunk per thread per row; a key row of DP elements spans CPR
 // threads, and a thread covers kPrepRows rows RPB apart (all loads first).
 constexpr int kPrepRows = 4;
-template <typename T, int DP>
+template <typename T, int DP, bool I8>
 __global__ __launch_bounds__(256) void prep_k_kernel(PrepKArgs a) {
   constexpr int VEC = 16 / (int)sizeof(T);
   constexpr int CPR = DP / VEC;  // chunks per row (power of two, <= 32)
@@ -390,6 +433,8 @@ __global__ __launch_bounds__(256) void prep_k_kernel(PrepKArgs a) {
   }
   const int bh = blockIdx.y - 1, b = bh / a.H, h = bh % a.H;
   const int d0 = (threadIdx.x % CPR) * VEC;
+  char* const khat = (char*)a.khat + (int64_t)bh * a.Tk_pad * DP * (int)sizeof(f16);  // the head's rows
+  const bool int8 = I8 && int8_window(a.w[h], a.Tq, a.Tk);
   float x[kPrepRows][VEC];
 #pragma unroll
   for (int u = 0; u < kPrepRows; ++u) {
@@ -402,21 +447,84 @@ __global__ __launch_bounds__(256) void prep_k_kernel(PrepKArgs a) {
       for (int e = 0; e < VEC; ++e) x[u][e] = 0.0f;
     }
   }
+  if (int8) {
+    // rows of the block: kPrepRows * RPB, whole units (a wave's rows lie in one)
+    constexpr int NU = kPrepRows * RPB / kUnit;
+    static_assert(!I8 || NU * kUnit == kPrepRows * RPB, "a block holds whole key units");
+    __shared__ unsigned umax[NU], uerr[NU];  // bits of non-negative floats: ordered as integers
+    if (threadIdx.x < NU) umax[threadIdx.x] = uerr[threadIdx.x] = 0u;
+    __syncthreads();
+    bool lost[kPrepRows];  // |k| too small for 1/|k| (eps = 0): the unit is marked whatever q is
 #pragma unroll
-  for (int u = 0; u < kPrepRows; ++u) {
-    const int64_t t = ((int64_t)blockIdx.x * kPrepRows + u) * RPB + threadIdx.x / CPR;
-    float ss = 0.0f;
+    for (int u = 0; u < kPrepRows; ++u) {
+      const int row = u * RPB + threadIdx.x / CPR;
+      const int64_t t = (int64_t)blockIdx.x * kPrepRows * RPB + row;
+      float ss = 0.0f, mx = 0.0f;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) ss += x[u][e] * x[u][e];
-    ss = group_sum<CPR>(ss);  // the row's CPR lanes
-    float inv = kKhatScale / fmaxf(sqrtf(ss), a.eps);
-    if (t >= a.Tk || (a.kpm != nullptr && a.kpm[(int64_t)b * a.Tk + t])) inv = 0.0f;
-    if (t < a.Tk_pad) {
-      ScreenOp* p = (ScreenOp*)a.khat + ((int64_t)bh * a.Tk_pad + t) * DP + d0;
+      for (int e = 0; e < VEC; ++e) ss += x[u][e] * x[u][e];
+      ss = group_sum<CPR>(ss);
+      float inv = 1.0f / fmaxf(sqrtf(ss), a.eps);
+      lost[u] = inv == INFINITY;
+      // padded and masked keys, and rows with no finite length: zero
+      const bool zero = t >= a.Tk || !(ss < INFINITY) || lost[u] ||
+                        (a.kpm != nullptr && a.kpm[(int64_t)b * a.Tk + t]);
+      lost[u] = lost[u] && t < a.Tk;
 #pragma unroll
-      for (int e = 0; e < VEC; e += 4)
-        store4(p + e, x[u][e] * inv, x[u][e + 1] * inv, x[u][e + 2] * inv, x[u][e + 3] * inv);
+      for (int e = 0; e < VEC; ++e) {
+        x[u][e] = zero ? 0.0f : x[u][e] * inv;
+        mx = fmaxf(mx, fabsf(x[u][e]));
+      }
+      atomicMax(&umax[row / kUnit], __float_as_uint(mx));
     }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPrepRows; ++u) {
+      const int row = u * RPB + threadIdx.x / CPR;
+      const int64_t t = (int64_t)blockIdx.x * kPrepRows * RPB + row;
+      const float mx = fmaxf(__uint_as_float(umax[row / kUnit]), 1e-30f), g = 127.0f / mx;
+      uint32_t q[VEC];
+      float se = 0.0f;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        float err;
+        q[e] = round_int8(x[u][e] * g, err);
+        se += err * err;
+      }
+      se = group_sum<CPR>(se);
+      if (threadIdx.x % CPR == 0)
+        atomicMax(&uerr[row / kUnit], __float_as_uint(lost[u] ? 4.0f : sqrtf(se) * mx * (1.0f / 127.0f)));
+      if (t < a.Tk_pad) {
+        // column 16a + 8b + c of a 32-column group is stored at 16b + 8a + c:
+        // a 16-byte chunk holds what a lane of the screen's query rows holds
+        uint32_t* p = (uint32_t*)(khat + t * DP + (d0 & ~31) + 16 * ((d0 >> 3) & 1) + 8 * ((d0 >> 4) & 1) +
+                                  (d0 & 7));
+#pragma unroll
+        for (int e = 0; e < VEC; e += 4) p[e / 4] = pack4(q[e], q[e + 1], q[e + 2], q[e + 3]);
+      }
+    }
+    __syncthreads();
+    const int64_t unit = (int64_t)blockIdx.x * NU + threadIdx.x, units = a.Tk_pad / kUnit;
+    if (threadIdx.x < NU && unit < units) {
+      const float g = 127.0f / fmaxf(__uint_as_float(umax[threadIdx.x]), 1e-30f);
+      ((KeyUnitScale*)(khat + a.Tk_pad * DP))[unit] = KeyUnitScale{g, __uint_as_float(uerr[threadIdx.x])};
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < kPrepRows; ++u) {
+      const int64_t t = ((int64_t)blockIdx.x * kPrepRows + u) * RPB + threadIdx.x / CPR;
+      float ss = 0.0f;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) ss += x[u][e] * x[u][e];
+      ss = group_sum<CPR>(ss);  // the row's CPR lanes
+      float inv = kKhatScale / fmaxf(sqrtf(ss), a.eps);
+      if (t >= a.Tk || (a.kpm != nullptr && a.kpm[(int64_t)b * a.Tk + t])) inv = 0.0f;
+      if (t < a.Tk_pad) {
+        f16* p = (f16*)khat + t * DP + d0;
+#pragma unroll
+        for (int e = 0; e < VEC; e += 4)
+          store4(p + e, x[u][e] * inv, x[u][e + 1] * inv, x[u][e + 2] * inv, x[u][e + 3] * inv);
+      }
+  }
   }
   // clear this head's live-tile bitmap rows; the screen ORs live bits in
   uint32_t* brow = a.bits + (int64_t)bh * a.bits_per_bh;
@@ -462,8 +570,10 @@ struct ScreenTile {
   static constexpr int TILEB = 64 * ROWB;            // bytes per staged key tile
   static constexpr int CPT = 64 * CPR / 256;         // DMA chunks per thread per tile
   // ring slots: the 4 tiles the waves read in a step plus the tiles in flight
-  // (2 for tiles up to 8 KiB: 48 KiB a block, three blocks a CU; 1 above)
-  static constexpr int NS = TILEB <= 8192 ? 6 : 5;
+  // (fp16: 2 for tiles up to 8 KiB, 48 KiB a block, three blocks a CU; 1 above.
+  // int8, whose steps are half as long: 6 for 4 KiB tiles, 4 for 8 KiB ones at
+  // two blocks a CU)
+  static constexpr int NS = sizeof(T) == 1 ? (TILEB <= 4096 ? 10 : 8) : (TILEB <= 8192 ? 6 : 5);
   // LDS chunk position of global chunk c of row R: c ^ swz(R), conflict-free
   // for the perm_row operand reads
   __device__ static inline int swz(int R) { return lds_swz<CPR>(R); }
@@ -489,18 +599,21 @@ __device__ inline int ceil_tiles(int x) { return -floor_tiles(-x); }
 // are ORed into the bitmap (cleared by prep_k_kernel), so items that share a
 // bitmap word need no ordering.
 // ---------------------------------------------------------------------------
-template <typename T, int DP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void fwd_screen_kernel(FwdKArgs a) {
-  using S = ScreenOp;  // operand type of the screen's MFMAs
-  using M = Mma<S>;
-  using frag = typename M::frag;
-  using G = ScreenTile<S, DP>;
-  constexpr int KS = M::KS, PER = M::PER, NKS = DP / KS, NS = G::NS;
-  __shared__ __attribute__((aligned(16))) char ring[NS * G::TILEB];
+template <typename T, int DP, bool ANY8>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DP == 128 ? 2 : 3, DP == 128 ? 2 : 3)))
+void fwd_screen_kernel(FwdKArgs a) {
+  constexpr int kRing16 = ScreenTile<f16, DP>::NS * ScreenTile<f16, DP>::TILEB;
+  constexpr int kRing8 = ScreenTile<int8_t, DP>::NS * ScreenTile<int8_t, DP>::TILEB;
+  // the ring; int8: behind it the scales of the item's key units, unit kh of
+  // tile number u at 2u + kh + 1 (one 16-byte read gives a step both it needs)
+  // (one array: with a second one the compiler waits for every copy in flight
+  // before each read)
+  constexpr int USN = 2 * (kScreenMaxSeg + 4);
+  constexpr int kBytes8 = kRing8 + USN * (int)sizeof(KeyUnitScale);
+  __shared__ __attribute__((aligned(16))) char ring[ANY8 && kBytes8 > kRing16 ? kBytes8 : kRing16];
 
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform values live in SGPRs
-  const int half = lane >> 5, l32 = lane & 31;
+  KeyUnitScale* const us = reinterpret_cast<KeyUnitScale*>(ring + kRing8);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);  // wave-uniform values live in SGPRs
   const int nkt = (int)(a.Tk_pad / kTile);
   // this block's lane: (XCD p % 8, engine (p >> 3) % 4); it runs the lane's
   // items at positions p >> 5, (p >> 5) + K, ... (K blocks per lane), which
@@ -514,8 +627,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   const int4 item = *(const int4*)(lane_items + pos);
   const float4 irw = *((const float4*)(lane_items + pos) + 1);
   asm volatile("" ::"v"(item.x), "v"(item.y), "v"(item.z), "v"(item.w), "v"(irw.x), "v"(irw.y));
-  if (item.x < 0) break;  // block-uniform: past this lane's items
-  const int bh = item.x, grp = item.y, olo = item.z, ohi = item.w;
+  // block-uniform, so kept in SGPRs
+  auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  const int bh = uni(item.x), grp = uni(item.y), olo = uni(item.z), ohi = uni(item.w);
+  if (bh < 0) break;  // past this lane's items
+  const float head_r = __int_as_float(uni(__float_as_int(irw.x)));
+  const float head_w = __int_as_float(uni(__float_as_int(irw.y)));
+  // the item on operands of type S, the head's
+  auto run = [&](auto op) __attribute__((always_inline)) {
+  using S = decltype(op);
+  using M = Mma<S>;
+  using Acc = typename M::acc;
+  constexpr bool I8 = __is_same(S, int8_t);
+  using frag = typename M::frag;
+  using G = ScreenTile<S, DP>;
+  constexpr int KS = M::KS, PER = M::PER, NKS = DP / KS, NS = G::NS;
+  uint32_t tid_opaque = threadIdx.x;
+  if constexpr (ANY8) rederive(tid_opaque);  // one operand type's offsets don't hold registers in the other's loops
+  const int tid = (int)tid_opaque, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
   const int b = bh / a.H, h = bh % a.H;
   const bool causal = a.causal != 0;
   const int qt = grp * 4 + wave;
@@ -534,14 +663,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   }
   __builtin_amdgcn_sched_barrier(0);  // query loads issue before the DMA
   frag qf[2 * NKS];
-  float qthr[2];  // vote threshold on acc for this lane's query of unit qh
+  float qthr[2];  // vote threshold on acc for this lane's query of unit qh (int8: A)
+  float qerr[2];  // int8: B
   // bitmap rows of the wave's two query units (32 queries each)
   uint32_t* brow = a.bits + ((int64_t)bh * 2 * a.nqt + 2 * (wave_ok ? qt : 0)) * a.nku_words;
 
   // DMA: chunk c = u*256 + tid of a tile (row c / CPR, LDS position c % CPR)
   // comes from global chunk position ^ swz(row) of that row; the per-lane
   // byte offset inside a tile is fixed, the tile base is uniform.
-  const char* kg = (const char*)a.khat + (int64_t)bh * a.Tk_pad * G::ROWB;
+  const char* kg = (const char*)a.khat + (int64_t)bh * a.Tk_pad * DP * (int)sizeof(f16);
   uint32_t goff[G::CPT];
 #pragma unroll
   for (int u = 0; u < G::CPT; ++u) {
@@ -568,11 +698,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
           (void __attribute__((address_space(3)))*)(ring + slot_idx * G::TILEB + (c * 256 + wave * 64) * 16), 16, 0,
           0);
   };
+  constexpr int NUS = (2 * (kScreenMaxSeg + 3) + 255) / 256;
+  KeyUnitScale usv[NUS];  // loads go before the DMA, so their wait leaves it in flight
+  if constexpr (I8) {
+#pragma unroll
+    for (int c = 0; c < NUS; ++c) {
+      if (c > 0 && c * 256 >= 2 * (nsteps + 3)) continue;  // block-uniform
+      int kt = A0 + (c * 256 + tid) / 2;
+      kt = kt < tmin ? tmin : (kt > tmax ? tmax : kt);
+      usv[c] = ((const KeyUnitScale*)(kg + a.Tk_pad * DP))[2 * kt + (tid & 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
 #pragma unroll
   for (int u = 0; u < NS - 1; ++u) issue(u, u);
   __builtin_amdgcn_sched_barrier(0);
 
-  const HeadParams hp = head_params_rw(irw.x, irw.y, causal);
+  const HeadParams hp = head_params_rw(head_r, head_w, causal);
   int kt_lo, kt_hi;
   key_tile_range(a, hp, causal, q0, q0 + 63 < a.Tq - 1 ? q0 + 63 : a.Tq - 1, kt_lo, kt_hi);
   if (!wave_ok) { kt_lo = 0; kt_hi = -1; }
@@ -590,14 +732,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     }
 
   // MFMAs of key half kh of the staged tile: acc[qh] = K^ rows 32kh + perm x Q^T
-  auto half_mma = [&](const char* slot, int kh, f32x16 (&acc)[2]) {
+  auto half_mma = [&](const char* slot, int kh, Acc (&acc)[2]) {
     frag kf[NKS];
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) kf[ks] = M::load((const S*)(slot + aoff[kh][ks]));
 #pragma unroll
     for (int qh = 0; qh < 2; ++qh)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[qh][r] = 0.0f;
+      for (int r = 0; r < 16; ++r) acc[qh][r] = 0;
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
@@ -618,22 +760,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // other tiles each 32x32 unit is classed by its distance range c-31 .. c+31
   // (the window is one interval of distances): wholly inside (plain maximum),
   // wholly outside (no vote) or cut by a window edge (per-register test).
-  auto vote_half = [&](const f32x16 (&acc)[2], int k0, int kh, bool interior) -> int {
+  auto vote_half = [&](const Acc (&acc)[2], int k0, int kh, bool interior, KeyUnitScale ku) -> int {
+    using E = typename M::acc_elem;
+    const E none = I8 ? (E)(-0x7fffffff - 1) : (E)(-INFINITY);
     int lv = 0;
 #pragma unroll
     for (int qh = 0; qh < 2; ++qh) {
-      float mx = -INFINITY;
+      E mx = none;
       const int c = q0 + 32 * qh - k0 - 32 * kh;  // wave-uniform
       if (interior || (in_window(c - 31, hp) && in_window(c + 31, hp))) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc[qh][r]);
+        for (int r = 0; r < 16; ++r) mx = M::max(mx, acc[qh][r]);
       } else if (c + 31 + hp.wsh >= 0 && c - 31 + hp.wsh < (int)hp.wlim) {
         const int rel0 = (q0 + 32 * qh + l32) - k0 - 32 * kh - 8 * half;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          mx = fmaxf(mx, in_window(rel0 - (16 * (r >> 3) + (r & 7)), hp) ? acc[qh][r] : -INFINITY);
+          mx = M::max(mx, in_window(rel0 - (16 * (r >> 3) + (r & 7)), hp) ? acc[qh][r] : none);
       }
-      lv |= (__ballot(mx > qthr[qh]) != 0ull ? 1 : 0) << qh;
+      if constexpr (I8) {
+        float t = ku.g * fmaf(-qerr[qh], ku.e, qthr[qh]);
+        if (!interior) t = fmaxf(t, -1e9f);  // |acc| < 2^21; `none` never passes
+        lv |= (__ballot((float)mx > t) != 0ull ? 1 : 0) << qh;
+      } else
+        lv |= (__ballot(mx > qthr[qh]) != 0ull ? 1 : 0) << qh;
     }
     return lv;
   };
@@ -682,7 +831,45 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   // acc > (1 - 1/r - slack) max(|q|, eps) c, with c = kKhatScale times the
   // row's power of two (a negative gate, r within the slack of 1, marks every
   // unit with a pair above it: still a superset of the live units)
-  {
+  if constexpr (I8) {
+    const float vthr = 1.0f - 1.0f / hp.r - kInt8Slack;
+#pragma unroll
+    for (int qh = 0; qh < 2; ++qh) {
+      float mx = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < 2 * NKS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(qrow[qh].get(ks, e)));
+      mx = half_max(mx);
+      const float inv = qrow[qh].inv_norm(a.eps);
+      // a row with no finite length (NaN leaves A = NaN) marks nothing
+      const bool dead = !(mx < INFINITY) || !(inv > 0.0f);
+      const float g = dead ? 0.0f : 127.0f / fmaxf(mx, 1e-30f);
+      float se = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < 2 * NKS; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+          uint32_t b4[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            float err;
+            b4[j] = round_int8(qrow[qh].get(ks, e + j) * g, err);
+            se += err * err;
+          }
+          qf[qh * NKS + ks / 2][2 * (ks & 1) + e / 4] = (int)pack4(b4[0], b4[1], b4[2], b4[3]);
+          __builtin_amdgcn_sched_barrier(0);  // few temporaries at a time
+        }
+      const float eq = sqrtf(half_sum(se)), N = g / inv;  // e_q N, g_q max(|q|, eps)
+      qthr[qh] = dead ? INFINITY : fmaf(vthr, N, -eq);
+      qerr[qh] = dead ? 0.0f : N + eq;
+    }
+    // the units' scales for every wave (the first step's barrier follows)
+#pragma unroll
+    for (int c = 0; c < NUS; ++c)
+      if ((c == 0 || c * 256 < 2 * (nsteps + 3)) && c * 256 + tid + 1 < USN) us[c * 256 + tid + 1] = usv[c];
+    wave_lds_sync();
+  } else {
     const float vthr = 1.0f - 1.0f / hp.r - kScreenSlack<T>;
 #pragma unroll
     for (int qh = 0; qh < 2; ++qh) {
@@ -708,7 +895,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     // one half runs while the MFMAs of the next half are in flight.  Order in
     // step n (this wave's tile kt): MFMA(kt, keys 0-31) -> finish tile kt-1
     // (vote on its keys 32-63) -> MFMA(kt, keys 32-63) -> vote(kt, keys 0-31).
-    f32x16 acc0[2], acc1[2];
+    Acc acc0[2], acc1[2];
+    // int8: scales of (tile u-1, keys 32-63) and (tile u, keys 0-31)
+    struct { KeyUnitScale prev, cur; } sc = {};
+    auto scales = [&](int u) {
+      if constexpr (I8) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(&us[2 * u]);
+        sc.prev = KeyUnitScale{v[0], v[1]};
+        sc.cur = KeyUnitScale{v[2], v[3]};
+      }
+    };
     bool pend = false, pint = false;  // tile kt-1: keys 32-63 pending in acc1
     int live0 = 0;                    // tile kt-1: vote on keys 0-31
     int pk0 = 0;
@@ -729,14 +925,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     // is outside its key range.
     auto step = [&](int n) {
       const char* slot = enter(n);
+      scales(n + wave);
       const int o = ohi - n, kt = A0 + n + wave;
       const bool mine = kt >= kt_lo && kt <= kt_hi;
       if (mine) half_mma(slot, 0, acc0);
-      if (n > 0 && pend) finish(kt - 1, live0, vote_half(acc1, pk0, 1, pint));
+      if (n > 0 && pend) finish(kt - 1, live0, vote_half(acc1, pk0, 1, pint, sc.prev));
       if (mine) {
         half_mma(slot, 1, acc1);
         pint = in_window(kTile * o + 63, hp) && in_window(kTile * o - 63, hp);
-        live0 = vote_half(acc0, kt * kTile, 0, pint);
+        live0 = vote_half(acc0, kt * kTile, 0, pint, sc.cur);
         pk0 = kt * kTile;
       }
       pend = mine;
@@ -747,10 +944,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     auto step_inside = [&](int n) {
       const char* slot = enter(n);
       const int kt = A0 + n + wave;
+      scales(n + wave);
       half_mma(slot, 0, acc0);
-      finish(kt - 1, live0, vote_half(acc1, 0, 1, true));
+      finish(kt - 1, live0, vote_half(acc1, 0, 1, true, sc.prev));
       half_mma(slot, 1, acc1);
-      live0 = vote_half(acc0, 0, 0, true);
+      live0 = vote_half(acc0, 0, 0, true, sc.cur);
       pend = true;
       pint = true;
       pk0 = kt * kTile;
@@ -759,13 +957,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     for (; n < n_fast0; ++n) step(n);
     for (; n < n_fast1; ++n) step_inside(n);
     for (; n < nsteps; ++n) step(n);
-    if (pend) finish(A0 + nsteps - 1 + wave, live0, vote_half(acc1, pk0, 1, pint));
+    if (pend) {
+      scales(nsteps + wave);
+      finish(A0 + nsteps - 1 + wave, live0, vote_half(acc1, pk0, 1, pint, sc.prev));
+    }
     // the trailing loads have landed and every wave is done with the ring
     // before the next item refills it
     wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
   }
   guard_frags(qf);
+  };
+  if constexpr (ANY8) {
+    if (int8_window(head_w, a.Tq, a.Tk)) run(int8_t());
+    else run(f16());
+  } else {
+    run(f16());
+  }
   }  // item loop
 }
 
@@ -785,7 +993,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // wave 0 through LDS, which adds them in wave order (fixed, so results repeat
 // bitwise) and runs the epilogue.
 // ---------------------------------------------------------------------------
-template <typename T, int DP, int S, bool DROP>
+// REFINE (after an int8 screen; S = 1, no dropout): a unit without a live pair
+// stops before its value product and loses its bit.
+template <typename T, int DP, int S, bool DROP, bool REFINE = false>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(unit_waves<T, DP>())))
 void fwd_live_kernel(FwdKArgs a) {
   using M = Mma<T>;
@@ -984,6 +1194,20 @@ void fwd_live_kernel(FwdKArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) body(r);
       }
+      // an int8 screen marks some units without a live pair: nothing of them
+      // reaches y or a gradient, and their bit is taken back (one wave walks
+      // a row when S = 1, and it holds the row's words already)
+      if constexpr (REFINE) {
+        float wmax = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) wmax = fmaxf(wmax, s[r]);
+        if (__ballot(wmax > 0.0f) == 0ull) {
+          if (lane == 0)
+            atomicAnd(a.bits + ((int64_t)bh * 2 * a.nqt + qu) * a.nku_words + (cur >> 5), ~(1u << (cur & 31)));
+          cur = nxt;
+          continue;
+        }
+      }
       __builtin_amdgcn_sched_barrier(0);
       float vsc[16];
       read_row_scales(sv, half, vsc);
@@ -1053,11 +1277,24 @@ void fwd_live_kernel(FwdKArgs a) {
   }
 }
 
+// A head's fp16 rows, or its int8 rows and then their units' scales.
 static int64_t khat_bytes(const Geometry& g) {
-  return round_up((int64_t)g.B * g.H * g.Tk_pad * g.DP * (int64_t)sizeof(ScreenOp), 256);  // fp16 rows
+  return round_up((int64_t)g.B * g.H * g.Tk_pad * g.DP * (int64_t)sizeof(f16), 256);
 }
 // Workspace: [K^][screen plan table]
 size_t fwd_ws_bytes(const Geometry& g) { return khat_bytes(g) + screen_plan_bytes(g); }
+
+// Whether heads of long windows screen on int8 operands (DP >= 64): 2-byte
+// inputs (an fp32 live pass spends more on a dead unit than the screen saves:
+// causal step T = 8192, B = 2: 277 -> 288 us), positions enough for a long
+// window, and a live pass of one wave a row without dropout, which takes the
+// dead units' bits back.
+template <typename T>
+static bool screens_int8(const FwdCall& c) {
+  const Geometry& g = c.g;
+  return sizeof(T) == 2 && !c.drop.on && (g.Tq > g.Tk ? g.Tq : g.Tk) >= kInt8Window &&
+         split_waves<T>((int64_t)2 * g.nqt * g.B * g.H) == 1;
+}
 
 template <typename T, int DP>
 static hipError_t launch_fwd_t(const FwdCall& c) {
@@ -1068,6 +1305,7 @@ static hipError_t launch_fwd_t(const FwdCall& c) {
   FwdKArgs fa;
   fa.q = c.q; fa.qs = c.qs; fa.k = c.k; fa.ks = c.ks; fa.v = c.v; fa.vs = c.vs; fa.kpm = c.kpm;
   fa.khat = c.khat;
+  const bool int8 = DP >= 64 && screens_int8<T>(c);
   fa.r = c.r; fa.w = c.w; fa.y = c.y; fa.hnorm = c.hnorm; fa.bits = c.bits;
   fa.H = g.H; fa.Tq = g.Tq; fa.Tk = g.Tk; fa.D = g.D; fa.nqt = g.nqt; fa.nku_words = g.nku_words;
   fa.causal = g.causal; fa.Tk_pad = g.Tk_pad; fa.eps = c.eps; fa.drop = c.drop;
@@ -1082,19 +1320,27 @@ static hipError_t launch_fwd_t(const FwdCall& c) {
     constexpr int RPB = 256 / (DP * (int)sizeof(T) / 16) * kPrepRows;
     const int64_t nx = (g.Tk_pad + RPB - 1) / RPB;
     // row 0: the screen planner (8 blocks); rows 1..B*H: K^ of head row-1
-    timer_begin(1, c.stream);
-    hipLaunchKernelGGL((prep_k_kernel<T, DP>), dim3((unsigned)(nx > 8 ? nx : 8), (unsigned)(g.B * g.H + 1)),
-                       dim3(256), 0, c.stream, pa);
-    timer_end(1, c.stream);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    timer_begin(2, c.stream);
+    const dim3 pgrid((unsigned)(nx > 8 ? nx : 8), (unsigned)(g.B * g.H + 1));
     // at most kScreenBlocksPerLane blocks per lane; blocks beyond the first
     // walk their lane's items with that stride
     const int per_lane = plan.kmax < kScreenBlocksPerLane ? plan.kmax : kScreenBlocksPerLane;
-    hipLaunchKernelGGL((fwd_screen_kernel<T, DP>), dim3((unsigned)(32 * per_lane)), dim3(256), 0, c.stream, fa);
-    timer_end(2, c.stream);
-    e = hipGetLastError();
+    auto screen = [&](auto any8) -> hipError_t {
+      constexpr bool A8 = decltype(any8)::value;
+      timer_begin(1, c.stream);
+      hipLaunchKernelGGL((prep_k_kernel<T, DP, A8>), pgrid, dim3(256), 0, c.stream, pa);
+      timer_end(1, c.stream);
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      timer_begin(2, c.stream);
+      hipLaunchKernelGGL((fwd_screen_kernel<T, DP, A8>), dim3((unsigned)(32 * per_lane)), dim3(256), 0, c.stream, fa);
+      timer_end(2, c.stream);
+      return hipGetLastError();
+    };
+    hipError_t e;
+    if constexpr (DP >= 64 && sizeof(T) == 2)
+      e = int8 ? screen(std::true_type{}) : screen(std::false_type{});
+    else
+      e = screen(std::false_type{});
     if (e != hipSuccess) return e;
   }
   // A launch with few rows (under about two waves per SIMD) splits each
@@ -1105,6 +1351,11 @@ static hipError_t launch_fwd_t(const FwdCall& c) {
   timer_begin(3, c.stream);
   auto launch = [&](auto drop) {
     constexpr bool DROP = decltype(drop)::value;
+    if constexpr (DP >= 64 && sizeof(T) == 2 && !DROP)
+      if (int8) {  // S = 1
+        hipLaunchKernelGGL((fwd_live_kernel<T, DP, 1, false, true>), grid, dim3(64), 0, c.stream, fa);
+        return;
+      }
     if (S == 4)
       hipLaunchKernelGGL((fwd_live_kernel<T, DP, 4, DROP>), grid, dim3(256), 0, c.stream, fa);
     else if (S == 2)
