@@ -11,7 +11,8 @@
 //                   global -> LDS by direct DMA into a ring (each tile is read
 //                   by the 4 waves in 4 consecutive steps).  Each wave forms
 //                   S^T = K^ Q^T on fp16 MFMA (the raw query rows rounded to
-//                   fp16, fp32 accumulation, scaled by 1/|q_i|) and votes whether any in-window pair passes the
+//                   fp16, fp32 accumulation; long windows of 2-byte inputs:
+//                   int8) and votes whether any in-window pair passes the
 //                   trim-and-square threshold (attention.py:75-90).  Output:
 //                   the live-unit bitmap (32x32 units).
 //   fwd_live_kernel : one wave per 32-query unit (S waves for launches with few
