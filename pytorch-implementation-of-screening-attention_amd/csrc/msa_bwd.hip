@@ -354,8 +354,12 @@ void dq_kernel(BwdKArgs a) {
     if (half == 0) {
       sk[m] = ikl;
       sv[m] = iv;
-      if constexpr (kPow2Rows<T>) {
-        const Pow2Split p(ikl);
+    }
+    bool two = false;  // fp16: some K row takes a second power of two
+    if constexpr (kPow2Rows<T>) {
+      const Pow2Split p(ikl);
+      two = p.two_factors();
+      if (half == 0) {
         sw_w[wave][m] = p.w;
         sc_w[wave][0][m] = (f16)p.c1;
         sc_w[wave][1][m] = (f16)p.c2;
@@ -418,13 +422,12 @@ void dq_kernel(BwdKArgs a) {
       for (int r = 0; r < 16; ++r) dp[r] *= ksc[r];
     }
     if constexpr (kPow2Rows<T>) {
-      const bool tiny = __ballot(ikl > 32768.0f) != 0ull;  // rows shorter than 2^-15
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int dblk = 0; dblk < NDH; ++dblk) {
           scale_slots(ka[dblk * NC + c], sc_w[wave][0], c, half);
-          if (tiny) scale_slots(ka[dblk * NC + c], sc_w[wave][1], c, half);
+          if (two) scale_slots(ka[dblk * NC + c], sc_w[wave][1], c, half);
         }
     }
     frag db[NC];
@@ -619,10 +622,12 @@ void dkdv_kernel(BwdKArgs a) {
     }
     wait_vmcnt<0>();  // the unit's rows have landed
     const float iqc = iqv;
-    if (half == 0) {
-      sq[l32] = iqc;
-      if constexpr (kPow2Rows<T>) {
-        const Pow2Split p(iqc);
+    if (half == 0) sq[l32] = iqc;
+    bool two = false;  // fp16: some Q row takes a second power of two
+    if constexpr (kPow2Rows<T>) {
+      const Pow2Split p(iqc);
+      two = p.two_factors();
+      if (half == 0) {
         sw_w[wave][l32] = p.w;
         sc_w[wave][0][l32] = (f16)p.c1;
         sc_w[wave][1][l32] = (f16)p.c2;
@@ -720,13 +725,12 @@ void dkdv_kernel(BwdKArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) dp[r] *= qsc[r];
     if constexpr (kPow2Rows<T>) {
-      const bool tiny = __ballot(iqc > 32768.0f) != 0ull;  // rows shorter than 2^-15
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int dblk = 0; dblk < NDH; ++dblk) {
           scale_slots(qa[dblk * NC + c], sc_w[wave][0], c, half);
-          if (tiny) scale_slots(qa[dblk * NC + c], sc_w[wave][1], c, half);
+          if (two) scale_slots(qa[dblk * NC + c], sc_w[wave][1], c, half);
         }
     }
     // dv^T[d][j] += sum_i dH^T[d][i] P[i][j];  dk^T[d][j] += sum_i Q^T[d][i] (ds/|q|)[i][j]

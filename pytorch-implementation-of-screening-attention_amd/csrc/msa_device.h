@@ -175,9 +175,9 @@ template <typename T>
 constexpr bool kPow2Rows = sizeof(T) == 2 && !__is_same(T, bf16);
 
 // The split of a row factor f = 1/|x| (0 for masked rows): w <= 1 and c = c1 c2,
-// each a power of two in fp16's normal range.  c2 is 1 except for rows
-// shorter than 2^-15; a zero row (f = 1/eps, past c's range) has w = 1 and
-// contributes its zeros whatever w is.  |x| > 2^14 leaves c at 2^-14.
+// each a power of two in fp16's normal range.  c2 differs from 1 for rows of
+// length 2^-15 and less (two_factors); a zero row (f = 1/eps, which may lie past
+// c's range) contributes its zeros whatever w is.  |x| > 2^14 leaves c at 2^-14.
 struct Pow2Split {
   float w, c1, c2;
   __device__ explicit Pow2Split(float f) {
@@ -186,6 +186,8 @@ struct Pow2Split {
     c2 = fminf(fmaxf(c * 3.0517578125e-5f, 1.0f), 32768.0f);             // c 2^-15
     w = fminf(f * recip(c1) * recip(c2), 1.0f);
   }
+  // Whether c2 has a part to play in some lane's row (wave-uniform).
+  __device__ inline bool two_factors() const { return __ballot(c2 != 1.0f) != 0ull; }
   __device__ static inline float recip(float p) { return __int_as_float(0x7f000000 - __float_as_int(p)); }  // 1/2^e
 };
 

@@ -1149,16 +1149,19 @@ void fwd_live_kernel(FwdKArgs a) {
       kmask = key_mask(nxt);
     }
     // 1/|k_j| and 1/|v_j| to LDS, read back in register order
-    if (half == 0) {
-      sk[m] = ik;
-      if constexpr (kPow2Rows<T>) {
-        const Pow2Split p(iv);
+    bool two = false;  // fp16: some V row takes a second power of two
+    if constexpr (kPow2Rows<T>) {
+      const Pow2Split p(iv);
+      two = p.two_factors();
+      if (half == 0) {
+        sk[m] = ik;
         sv[m] = p.w;
         sc_w[wave][0][m] = (f16)p.c1;
         sc_w[wave][1][m] = (f16)p.c2;
-      } else {
-        sv[m] = iv;
       }
+    } else if (half == 0) {
+      sk[m] = ik;
+      sv[m] = iv;
     }
     unit_mask_table<false>(mt, nullptr, qu * kUnit - k0 - 31, hp, lane);
     wave_lds_sync();
@@ -1216,14 +1219,12 @@ void fwd_live_kernel(FwdKArgs a) {
       for (int r = 0; r < 16; ++r) s[r] *= vsc[r];
     }
     if constexpr (kPow2Rows<T>) {
-      // c2 differs from 1 only for rows shorter than 2^-15
-      const bool tiny = __ballot(iv > 32768.0f) != 0ull;
 #pragma unroll
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int dblk = 0; dblk < NDH; ++dblk) {
           scale_slots(va[dblk * NC + c], sc_w[wave][0], c, half);
-          if (tiny) scale_slots(va[dblk * NC + c], sc_w[wave][1], c, half);
+          if (two) scale_slots(va[dblk * NC + c], sc_w[wave][1], c, half);
         }
     }
     // H^T[d][i] += sum_j V^T[d][j] P^T[j][i]
