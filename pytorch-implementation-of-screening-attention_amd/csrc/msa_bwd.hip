@@ -66,7 +66,9 @@ struct BwdKArgs {
   const uint32_t* bits;
   void* dq; void* dk; void* dv; float* dr; float* dw;
   float* part;  // workspace: (dr, dw) shares per (b, h, query unit), [2][b*h][2*nqt]
-  void* dh; float* iqs;  // workspace: dh [b*h][Tq_pad][DP] (T), 1/|q| [b*h][Tq_pad]
+  // workspace: dh [b*h][Tq_pad][DP] (T), 1/|q| [b*h][Tq_pad] (fp16: negative for
+  // rows whose ds may come within a factor 2 of fp16's range)
+  void* dh; float* iqs;
   int B, H, Tq, Tk, D, nqt, nkt, nku_words, causal;
   int64_t Tq_pad;
   float eps;
@@ -266,6 +268,11 @@ void dq_kernel(BwdKArgs a) {
   // own queries' rows first, then the first key unit's copies behind them
   frag qf[NKS];  // raw q operand fragments; those of dh are kept in LDS (read back per unit)
   float iql;
+  // fp16: dh's row enters as dh p, p the power of two that makes its largest
+  // element (times the dropout scale) 2^10 .. 2^11.  The packed ds (without 2r)
+  // is then at most 2 * 2^11 sqrt(D) < 2^16, and the row's whole range has
+  // fp16's full precision however small or large the gradient is.
+  float ip = 1.0f;  // 1/p
   unsigned kmask = 0u;
   {
     QueryRows<T, DP> qr;
@@ -276,15 +283,35 @@ void dq_kernel(BwdKArgs a) {
       kmask = key_mask(cur);
     }
     iql = qr.finish(a.eps);
+    float p = 1.0f;
+    bool big = false;  // 2r a m dP w, w < 2, may leave fp16's range
+    if constexpr (kPow2Rows<T>) {
+      float mx = 0.0f;
+#pragma unroll
+      for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+        for (int e = 0; e < PER; ++e) mx = fmaxf(mx, fabsf(qr.dh.get(ks, e)));
+      mx = half_max(mx) * (DROP ? a.drop.scale : 1.0f);
+      p = row_pow2(mx);
+      ip = 1.0f / p;
+      big = !(4.0f * hp.r * mx * (DP == 128 ? 11.32f : (DP == 64 ? 8.0f : 5.66f)) < 65504.0f);  // |dP| <= sqrt(D) mx
+    }
     // dh and 1/|q| of this unit's rows for dkdv_kernel (zero past Tq)
     T* dst = (T*)a.dh + ((int64_t)bh * a.Tq_pad + i) * DP;
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
       qf[ks] = qr.q.f[ks];
-      hsh[ks][lane] = qr.dh.f[ks];
       if (wave == 0) *reinterpret_cast<frag*>(dst + KS * ks + PER * half) = qr.dh.f[ks];
+      if constexpr (kPow2Rows<T>) {
+        f32x16 t;
+#pragma unroll
+        for (int e = 0; e < PER; ++e) t[e] = qr.dh.get(ks, e) * p;
+        hsh[ks][lane] = M::pack(t, 0);
+      } else {
+        hsh[ks][lane] = qr.dh.f[ks];
+      }
     }
-    if (wave == 0 && half == 0) a.iqs[(int64_t)bh * a.Tq_pad + i] = valid ? iql : 0.0f;
+    if (wave == 0 && half == 0) a.iqs[(int64_t)bh * a.Tq_pad + i] = !valid ? 0.0f : (big ? -iql : iql);
   }
   const float thq = hp.thr / iql;  // s > thr  <=>  (q . k)/|k| > thr |q|
   const float riq = hp.r * iql;
@@ -441,8 +468,8 @@ void dq_kernel(BwdKArgs a) {
     guard_keep(db);
     cur = nxt;
   }
-  dr_acc = wave_sum(dr_acc) * (-2.0f / hp.r);
-  dw_acc = wave_sum(dw_acc);
+  dr_acc = wave_sum(dr_acc * ip) * (-2.0f / hp.r);
+  dw_acc = wave_sum(dw_acc * ip);
   if constexpr (S > 1) {
     auto part = [&](int w) { return reinterpret_cast<float(*)[kWave]>(stage[w]); };
     if (wave > 0) {
@@ -466,7 +493,7 @@ void dq_kernel(BwdKArgs a) {
 #pragma unroll
   for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) adq[dblk][r] *= 2.0f * hp.r;
+    for (int r = 0; r < 16; ++r) adq[dblk][r] *= 2.0f * hp.r * ip;
   zero_past_d<T, DP>(adq, a.D);
   write_norm_bwd<T, DP>(adq, qf, valid, a.D, a.eps, half, dqrow());
   if (lane == 0) {
@@ -606,6 +633,10 @@ void dkdv_kernel(BwdKArgs a) {
     iqv = iq0[(int64_t)cur * kUnit + l32];  // lanes l and l+32 read the same row
   }
   kr.finish(a.eps, ikl, ivl);
+  // what dp takes of the key's side: 2r/|v|, in the epilogue; in fp16 before ds is
+  // packed, as small gradients would be subnormal there without 2r and large ones
+  // out of range without 1/|v|
+  const float kfac = 2.0f * hp.r * ivl;
   f32x16 acc_k[NDH], acc_v[NDH];
 #pragma unroll
   for (int dblk = 0; dblk < NDH; ++dblk)
@@ -621,11 +652,10 @@ void dkdv_kernel(BwdKArgs a) {
       rederive(cb);
     }
     wait_vmcnt<0>();  // the unit's rows have landed
-    const float iqc = iqv;
-    if (half == 0) sq[l32] = iqc;
+    if (half == 0) sq[l32] = kPow2Rows<T> ? fabsf(iqv) : iqv;
     bool two = false;  // fp16: some Q row takes a second power of two
     if constexpr (kPow2Rows<T>) {
-      const Pow2Split p(iqc);
+      const Pow2Split p(iqv);
       two = p.two_factors();
       if (half == 0) {
         sw_w[wave][l32] = p.w;
@@ -682,14 +712,13 @@ void dkdv_kernel(BwdKArgs a) {
     } else {
       wave_lds_sync();
     }
-    // scaled in place: s = (q . k)/|q|; dp = dh . v takes its lane's 1/|v| and
-    // 2r once, in the epilogue (fp16: 1/|v| here, to keep ds in range)
+    // scaled in place: s = (q . k)/|q|; dp = dh . v, in fp16 with kfac
     float qsc[16];
     read_row_scales(sq, half, qsc);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       scale_pair<T>(s, slo, r, qsc[r]);
-      if constexpr (kPow2Rows<T>) dp[r] *= ivl;
+      if constexpr (kPow2Rows<T>) dp[r] *= kfac;
     }
     __builtin_amdgcn_sched_barrier(0);
     // every lane forms its pair's weight and ds branch-free (the mask, 0
@@ -797,7 +826,7 @@ void dkdv_kernel(BwdKArgs a) {
 #pragma unroll
   for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc_k[dblk][r] *= kPow2Rows<T> ? 2.0f * hp.r : 2.0f * hp.r * ivl;
+    for (int r = 0; r < 16; ++r) acc_k[dblk][r] *= kPow2Rows<T> ? 1.0f : kfac;
   zero_past_d<T, DP>(acc_k, a.D);
   zero_past_d<T, DP>(acc_v, a.D);
   write_norm_bwd<T, DP>(acc_k, kr.k.f, jvalid, a.D, a.eps, half, (T*)a.dk + orow);

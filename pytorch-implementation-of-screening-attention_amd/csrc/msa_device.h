@@ -169,27 +169,41 @@ template <> struct Mma<f16> {
 // pair weights (alpha*m/|v|, ds/|k|, ds/|q|) and keep the raw rows exact.
 // fp16 has 5 exponent bits: a weight times 1/|x| overflows to inf for rows
 // shorter than about 1.5e-5 (a zero row gives 1/eps = 1e8, then inf * 0 =
-// NaN).  There 1/|x| = c w with c a power of two and w in [1/2, 1]: the rows
+// NaN).  There 1/|x| = c w with c a power of two and w in [1, 2): the rows
 // take c, which only moves their exponent, and the weights take w.
 template <typename T>
 constexpr bool kPow2Rows = sizeof(T) == 2 && !__is_same(T, bf16);
 
-// The split of a row factor f = 1/|x| (0 for masked rows): w <= 1 and c = c1 c2,
-// each a power of two in fp16's normal range.  c2 differs from 1 for rows of
-// length 2^-15 and less (two_factors); a zero row (f = 1/eps, which may lie past
-// c's range) contributes its zeros whatever w is.  |x| > 2^14 leaves c at 2^-14.
+// The split of a row factor f = 1/|x| (0 for masked rows): w in [1, 2), so a
+// weight packed with it never has fewer bits than without, and c = c1 c2, each a
+// power of two that fp16 holds (c >= 2^-20 for any fp16 row).  The split of -f
+// has w in [1/2, 1), for weights that may lie within a factor 2 of fp16's range.
+// c2 differs from 1 for short rows (two_factors); a zero row (f = 1/eps, which may
+// lie past c's range) contributes its zeros whatever w is.
 struct Pow2Split {
   float w, c1, c2;
   __device__ explicit Pow2Split(float f) {
-    const float c = __int_as_float((__float_as_int(f) & 0x7f800000) + 0x00800000);
-    c1 = fminf(fmaxf(c, 6.103515625e-5f), 32768.0f);                    // 2^-14 .. 2^15
+    const uint32_t b = __float_as_uint(f);
+    const float c = __uint_as_float((b & 0x7f800000u) + ((b & 0x80000000u) >> 8));
+    c1 = fminf(fmaxf(c, 5.9604644775390625e-8f), 32768.0f);              // 2^-24 .. 2^15
     c2 = fminf(fmaxf(c * 3.0517578125e-5f, 1.0f), 32768.0f);             // c 2^-15
-    w = fminf(f * recip(c1) * recip(c2), 1.0f);
+    w = fminf(fabsf(f) * recip(c1) * recip(c2), 2.0f);
   }
   // Whether c2 has a part to play in some lane's row (wave-uniform).
   __device__ inline bool two_factors() const { return __ballot(c2 != 1.0f) != 0ull; }
   __device__ static inline float recip(float p) { return __int_as_float(0x7f000000 - __float_as_int(p)); }  // 1/2^e
 };
+
+// Power of two p with max|x| * p in [2^10, 2^11) (1 for a zero or non-finite
+// max): scales a row into fp16's normal range exactly.
+__device__ inline float row_pow2(float mx) {
+  if (!(mx > 0.0f) || !(mx < INFINITY)) return 1.0f;
+  int ex;
+  (void)frexpf(mx, &ex);  // mx = m 2^ex, m in [0.5, 1)
+  int e = 11 - ex;
+  e = e > 126 ? 126 : (e < -126 ? -126 : e);
+  return ldexpf(1.0f, e);
+}
 
 // fp32: a fragment is four v_mfma_f32_32x32x2_f32 steps, step e contracting the
 // lanes' slot e (half 0: column 8ks + e, half 1: column 8ks + 4 + e), so a

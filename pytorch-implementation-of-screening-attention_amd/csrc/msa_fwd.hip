@@ -383,17 +383,6 @@ struct WideQueryRow {
 template <typename T, int DP>
 using ScreenQueryRow = typename std::conditional<sizeof(T) == 2, PRow<T, DP>, WideQueryRow<DP>>::type;
 
-// Power of two p with max|x| * p in [2^10, 2^11) (1 for a zero or non-finite
-// max): scales a query row into fp16's normal range exactly.
-__device__ inline float row_pow2(float mx) {
-  if (!(mx > 0.0f) || !(mx < INFINITY)) return 1.0f;
-  int ex;
-  (void)frexpf(mx, &ex);  // mx = m 2^ex, m in [0.5, 1)
-  int e = 11 - ex;
-  e = e > 126 ? 126 : (e < -126 ? -126 : e);
-  return ldexpf(1.0f, e);
-}
-
 // int8 of y (|y| <= 127, in its low byte) and the rounding's error y - round(y).
 __device__ inline uint32_t round_int8(float y, float& err) {
   const float f = y + 12582912.0f;  // 1.5 * 2^23: the sum's low bits are round(y)
@@ -1151,7 +1140,7 @@ void fwd_live_kernel(FwdKArgs a) {
     // 1/|k_j| and 1/|v_j| to LDS, read back in register order
     bool two = false;  // fp16: some V row takes a second power of two
     if constexpr (kPow2Rows<T>) {
-      const Pow2Split p(iv);
+      const Pow2Split p(DROP && a.drop.scale > 32000.0f ? -iv : iv);
       two = p.two_factors();
       if (half == 0) {
         sk[m] = ik;

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import screening_oracle as O
-from helpers import np64, rel_err, rw64
+from helpers import errors, head_sum_err, np64, rel_err, rw64
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +50,36 @@ def test_rows_around_two_to_the_minus_15(short, B):
         e = rel_err(got, want)
         print(f"fp16 rows {short} B={B} {name}: rel err {e:.3e}", flush=True)
         assert e <= TOL, f"{name}: rel err {e:.3e} > {TOL}"
+
+
+@pytest.mark.parametrize("B", [1, 40], ids=["shared_rows", "one_wave_a_row"])
+@pytest.mark.parametrize("dy_rms,r,size", [(1e-5, [8.0, 30.0], 2.0 ** -9), (2000.0, [2.0, 4.0], 1.0)],
+                         ids=["small_dy", "large_dy"])
+def test_gradients_at_the_ends_of_the_range(dy_rms, r, size, B):
+    """ds = 2 r a m dP is an fp16 operand of dq and dk.  At dy about 1e-5 the
+    plain product a m dP is about 1e-6, 17 of fp16's smallest steps (a step is
+    6e-8, so its rounding is 2% of it); 2r takes it out of there.  What is left
+    is dh's own rounding to fp16: 0.29 steps of 168, 2e-3.  At dy about 2000
+    the largest ds is above 32752, where another factor 2 is past the range.
+    q, k and v are short for the small dy, so that dq, dk and dv are not."""
+    from multiscreen import ops
+    T, H, D = 160, 2, 64
+    w = [24.0, 40.0]
+    g = torch.Generator().manual_seed(5)
+    centre = torch.randn(1, 1, H, D, generator=g)
+    noise = torch.tensor([(0.6 / x) ** 0.5 for x in r]).view(1, 1, H, 1)  # 1 - s about 0.6/r, a about 0.4
+    q, k = ((size * (centre + noise * torch.randn(B, T, H, D, generator=g))).half() for _ in range(2))
+    v = (size * torch.randn(B, T, H, D, generator=g)).half()
+    dy = (dy_rms * torch.randn(B, T, H, D, generator=g)).half()
+    rg, wg = torch.tensor(r, device=DEV), torch.tensor(w, device=DEV)
+    args = [t.to(DEV) for t in (q, k, v)]
+    y, hnorm, bits = ops.fwd_raw(*args, rg, wg, True, 1e-8, None)
+    grads = ops.bwd_raw(*args, rg, wg, True, 1e-8, y, hnorm, bits, dy.to(DEV))
+    _, ref, P = O.sparse_forward_backward(np64(q), np64(k), np64(v), rw64(r), rw64(w), np64(dy), True)
+    for name, got, want in zip(("dq", "dk", "dv"), grads, ref):
+        e = errors(np64(got), want)
+        print(f"fp16 dy {dy_rms} B={B} {name}: {e['max']:.3e} {e['fro']:.3e}", flush=True)
+        assert e["max"] <= TOL and e["fro"] <= TOL, f"{name}: {e}"
+    for name, got, want, scale in (("dr", grads[3], ref[3], P["dr_abs"]), ("dw", grads[4], ref[4], P["dw_abs"])):
+        e = head_sum_err(np64(got), want, scale)
+        assert e <= TOL, f"{name}: per-head error {e:.3e}"
