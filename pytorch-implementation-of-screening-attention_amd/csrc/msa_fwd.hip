@@ -983,8 +983,9 @@ void fwd_screen_kernel(FwdKArgs a) {
 // wave 0 through LDS, which adds them in wave order (fixed, so results repeat
 // bitwise) and runs the epilogue.
 // ---------------------------------------------------------------------------
-// REFINE (after an int8 screen; S = 1, no dropout): a unit without a live pair
-// stops before its value product and loses its bit.
+// REFINE (after an int8 screen; S = 1, no dropout): a unit whose pairs all lie
+// below the threshold, beyond the rounding of s, stops before its pair weights
+// and loses its bit.
 template <typename T, int DP, int S, bool DROP, bool REFINE = false>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(unit_waves<T, DP>())))
 void fwd_live_kernel(FwdKArgs a) {
@@ -1170,6 +1171,31 @@ void fwd_live_kernel(FwdKArgs a) {
     // there only
     {
       const float* mrow = mt + (l32 - 8 * half + 8);  // entry 23 - (16(r/8) + r%8): a constant offset
+      // an int8 screen marks some units without a live pair: nothing of them
+      // reaches y or a gradient, and their bit is taken back (one wave walks a
+      // row when S = 1, and it holds the row's words already).  A unit stays if
+      // some in-window pair passes the conservative gate: a pair that is live by
+      // less than the rounding of s keeps its unit marked.
+      if constexpr (REFINE) {
+        float smax = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) smax = fmaxf(smax, s[r]);
+        bool keep = __ballot(smax > thq) != 0ull;
+        const int c = qu * kUnit - k0;
+        if (keep && !(in_window(c - 31, hp) && in_window(c + 31, hp))) {  // a window edge cuts the unit
+          smax = -INFINITY;
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            smax = mrow[23 - (16 * (r >> 3) + (r & 7))] > 0.0f ? fmaxf(smax, s[r]) : smax;
+          keep = __ballot(smax > thq) != 0ull;
+        }
+        if (!keep) {
+          if (lane == 0)
+            atomicAnd(a.bits + ((int64_t)bh * 2 * a.nqt + qu) * a.nku_words + (cur >> 5), ~(1u << (cur & 31)));
+          cur = nxt;
+          continue;
+        }
+      }
       auto body = [&](int r) {
         const int off = 16 * (r >> 3) + (r & 7);
         const float av = pair_root<T>(s[r], slo[r], iq, riq, hp.r);
@@ -1186,20 +1212,6 @@ void fwd_live_kernel(FwdKArgs a) {
       } else {
 #pragma unroll
         for (int r = 0; r < 16; ++r) body(r);
-      }
-      // an int8 screen marks some units without a live pair: nothing of them
-      // reaches y or a gradient, and their bit is taken back (one wave walks
-      // a row when S = 1, and it holds the row's words already)
-      if constexpr (REFINE) {
-        float wmax = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) wmax = fmaxf(wmax, s[r]);
-        if (__ballot(wmax > 0.0f) == 0ull) {
-          if (lane == 0)
-            atomicAnd(a.bits + ((int64_t)bh * 2 * a.nqt + qu) * a.nku_words + (cur >> 5), ~(1u << (cur & 31)));
-          cur = nxt;
-          continue;
-        }
       }
       __builtin_amdgcn_sched_barrier(0);
       float vsc[16];

@@ -87,3 +87,29 @@ def test_int8_screen_marks_the_live_units(dtype, D, Tq, Tk, causal, padded):
                                               key_padding_mask=kp, pairs=live)
     assert rel_err(np64(y), yref) <= 2e-2
     assert rel_err(np64(grads[2]), gref[2]) <= 2e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+def test_pairs_at_the_threshold_keep_their_unit(dtype):
+    """Each head's r is the largest fp32 value at which its most similar pair is
+    live in float64 (a = 1 - r(1 - s) below 2e-7): the fp32 a of such a pair is
+    as often 0 as not, and its unit stays marked either way."""
+    from multiscreen import ops
+    T, H, D = 4096, 16, 64
+    for seed in range(3):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        q, k, v = (torch.randn(1, T, H, D, device=DEV, generator=g).to(dtype) for _ in range(3))
+        later = torch.ones(T, T, dtype=torch.bool, device=DEV).triu(1)
+        r, at = [], []
+        for h in range(H):
+            qh, kh = (torch.nn.functional.normalize(x[0, :, h].double(), dim=-1) for x in (q, k))
+            s = (qh @ kh.T).masked_fill_(later, -1.0)
+            at.append(divmod(int(s.argmax()), T))
+            bound = 1.0 / (1.0 - float(s.max()))
+            x = np.float32(bound)
+            r.append(float(x if x < bound else np.nextafter(x, np.float32(0))))
+        rg, wg = torch.tensor(r, device=DEV), torch.full((H,), 1e5, device=DEV)
+        y, hnorm, bits = ops.fwd_raw(q, k, v, rg, wg, True, 1e-8, None)
+        units = _units(bits, 1, H, T, T)
+        missed = [h for h, (i, j) in enumerate(at) if not units[0, h, i // 32, j // 32]]
+        assert not missed, f"heads {missed} of {H}: the unit of the live pair is not marked"
