@@ -314,7 +314,6 @@ void dq_kernel(BwdKArgs a) {
     if (wave == 0 && half == 0) a.iqs[(int64_t)bh * a.Tq_pad + i] = !valid ? 0.0f : (big ? -iql : iql);
   }
   const float thq = hp.thr / iql;  // s > thr  <=>  (q . k)/|k| > thr |q|
-  const float riq = hp.r * iql;
   float dr_acc = 0.0f, dw_acc = 0.0f;  // this unit's share of dr, dw
   f32x16 adq[NDH];
 #pragma unroll
@@ -419,7 +418,7 @@ void dq_kernel(BwdKArgs a) {
       // = -2 um (1 - s) = -(2/r) um (1 - a), dw = a^2 dP dm/dw
       auto body = [&](int r) {
         const int off = 16 * (r >> 3) + (r & 7);
-        const float av = pair_root<T>(s[r], slo[r], iql, riq, hp.r);
+        const float av = pair_root<T>(s[r], slo[r], iql, hp.r);
         float u = av * dp[r];
         if constexpr (DROP) u *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
         const float um = u * mrow[23 - off];
@@ -642,7 +641,6 @@ void dkdv_kernel(BwdKArgs a) {
   for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { acc_k[dblk][r] = 0.0f; acc_v[dblk][r] = 0.0f; }
-  const float rik = hp.r * ikl;
   const float thk = hp.thr / ikl;  // s > thr  <=>  (q . k)/|q| > thr |k|  (+inf for masked keys)
 
   while (cur >= 0) {
@@ -730,7 +728,7 @@ void dkdv_kernel(BwdKArgs a) {
       const float* mrow = mt + (8 * half - l32 + 31);
       auto body = [&](int r) {
         const int off = 16 * (r >> 3) + (r & 7);
-        const float av = pair_root<T>(s[r], slo[r], ikl, rik, hp.r);
+        const float av = pair_root<T>(s[r], slo[r], ikl, hp.r);
         float mk = mrow[off];
         if constexpr (DROP) mk *= dropout_factor(a.drop, bh, q0 + 8 * half + off, j);
         const float am = av * mk;

@@ -1080,7 +1080,6 @@ void fwd_live_kernel(FwdKArgs a) {
   }
   const float iq = qr.inv_norm(a.eps);
   const float thq = hp.thr / iq;  // s > thr  <=>  (k . q)/|k| > thr |q|
-  const float riq = hp.r * iq;
   f32x16 o[NDH];
 #pragma unroll
   for (int dblk = 0; dblk < NDH; ++dblk)
@@ -1198,7 +1197,7 @@ void fwd_live_kernel(FwdKArgs a) {
       }
       auto body = [&](int r) {
         const int off = 16 * (r >> 3) + (r & 7);
-        const float av = pair_root<T>(s[r], slo[r], iq, riq, hp.r);
+        const float av = pair_root<T>(s[r], slo[r], iq, hp.r);
         float p = av * av * mrow[23 - off];
         if constexpr (DROP) p *= dropout_factor(a.drop, bh, i, k0 + 8 * half + off);
         s[r] = p;
