@@ -392,6 +392,19 @@ void dq_kernel(BwdKArgs a) {
       }
     }
     wave_lds_sync();
+    // the K columns' second power of two, rarely needed.  At D <= 32 it is branched
+    // off here, where few values are live: beside the first one, below, the branch
+    // splits the straight-line part and 22 registers spill (three waves a SIMD),
+    // 149 -> 98 us at B=4 T=2048; D = 64 takes 148 us either way, D = 128 169
+    // here and 165 below.
+    auto scale_cols = [&](auto p) {  // fp16 only
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int dblk = 0; dblk < NDH; ++dblk) scale_slots(ka[dblk * NC + c], sc_w[wave][p], c, half);
+    };
+    if constexpr (kPow2Rows<T> && DP == 32)
+      if (two) scale_cols(1);
     // scaled in place: s = (q . k)/|k|, dp = dH . v^
     {
       float sc[16];
@@ -448,13 +461,8 @@ void dq_kernel(BwdKArgs a) {
       for (int r = 0; r < 16; ++r) dp[r] *= ksc[r];
     }
     if constexpr (kPow2Rows<T>) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int dblk = 0; dblk < NDH; ++dblk) {
-          scale_slots(ka[dblk * NC + c], sc_w[wave][0], c, half);
-          if (two) scale_slots(ka[dblk * NC + c], sc_w[wave][1], c, half);
-        }
+      scale_cols(0);
+      if (DP > 32 && two) scale_cols(1);
     }
     frag db[NC];
 #pragma unroll

@@ -1154,6 +1154,19 @@ void fwd_live_kernel(FwdKArgs a) {
     }
     unit_mask_table<false>(mt, nullptr, qu * kUnit - k0 - 31, hp, lane);
     wave_lds_sync();
+    // the V columns' second power of two, rarely needed.  At D >= 64 it is branched
+    // off here, where few values are live: beside the first one, below, the branch
+    // splits the straight-line part and registers spill (B=2 T=500 D=64 12.6 ->
+    // 11.1 us, B=4 T=2048 D=128 133 -> 120); D = 32 has the registers (B=4
+    // T=2048 78 us here, 70 below).
+    auto scale_cols = [&](auto p) {  // fp16 only
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int dblk = 0; dblk < NDH; ++dblk) scale_slots(va[dblk * NC + c], sc_w[wave][p], c, half);
+    };
+    if constexpr (kPow2Rows<T> && DP > 32)
+      if (two) scale_cols(1);
     {
       float ksc[16];
       read_row_scales(sk, half, ksc);
@@ -1219,13 +1232,8 @@ void fwd_live_kernel(FwdKArgs a) {
       for (int r = 0; r < 16; ++r) s[r] *= vsc[r];
     }
     if constexpr (kPow2Rows<T>) {
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int dblk = 0; dblk < NDH; ++dblk) {
-          scale_slots(va[dblk * NC + c], sc_w[wave][0], c, half);
-          if (two) scale_slots(va[dblk * NC + c], sc_w[wave][1], c, half);
-        }
+      scale_cols(0);
+      if (DP == 32 && two) scale_cols(1);
     }
     // H^T[d][i] += sum_j V^T[d][j] P^T[j][i]
     frag pb[NC];
