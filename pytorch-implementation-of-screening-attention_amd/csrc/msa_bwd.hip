@@ -177,6 +177,17 @@ __device__ inline void write_norm_bwd(const f32x16 (&acc)[DP / 32], const typena
 // ---------------------------------------------------------------------------
 template <typename T, int DP>
 constexpr int dq_waves() { return sizeof(T) * DP <= 64 ? 3 : (sizeof(T) * DP <= 128 ? 2 : 1); }
+// fp32 rows of D = 128: the K columns are read from the staged rows only where
+// they are used, and K's next copy waits for that; held across the pair terms as
+// in the other cases they spill 68 registers, and each reload waits behind the
+// copies in flight.  With one or two waves a row the dh fragments stay in
+// registers too, so that a CU's LDS holds four waves instead of three or two;
+// four waves a row fit it once either way and share the copy in LDS.  us a
+// launch, columns held -> columns late -> dh in registers too: B=4 H=8, T=4096
+// (one wave) 4257 -> 2531 -> 2256, T=2048 (two) 1542 -> 1134 -> 687, T=1000 (four)
+// 412 -> 239 -> 258.
+template <typename T, int DP>
+constexpr bool kLateK = sizeof(T) * DP > 256;
 
 template <typename T, int DP, int S, bool DROP>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(dq_waves<T, DP>())))
@@ -193,7 +204,8 @@ void dq_kernel(BwdKArgs a) {
   __shared__ __attribute__((aligned(16))) f16 sc_w[kPow2Rows<T> ? S : 1][2][32];  // fp16: its powers of two
   __shared__ __attribute__((aligned(1024))) char stage[S][2 * U::BYTES];  // the unit's K and V rows; then the partial dq
   static_assert(NDH * 16 * kWave * 4 <= 2 * U::BYTES, "the partial dq fits the staged rows");
-  __shared__ frag hsh[NKS][kWave];  // own dh operand fragments (each wave writes the same ones)
+  constexpr bool kDhRegs = kLateK<T, DP> && S < 4;
+  __shared__ frag hsh[kDhRegs ? 1 : NKS][kWave];  // own dh operand fragments (each wave writes the same ones)
   const int lane = (int)(threadIdx.x & 63), half = lane >> 5, l32 = lane & 31;
   const int wave = S > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
   float* sk = sk_w[wave];
@@ -267,6 +279,7 @@ void dq_kernel(BwdKArgs a) {
 
   // own queries' rows first, then the first key unit's copies behind them
   frag qf[NKS];  // raw q operand fragments; those of dh are kept in LDS (read back per unit)
+  frag hreg[kDhRegs ? NKS : 1];
   float iql;
   // fp16: dh's row enters as dh p, p the power of two that makes its largest
   // element (times the dropout scale) 2^10 .. 2^11.  The packed ds (without 2r)
@@ -307,6 +320,8 @@ void dq_kernel(BwdKArgs a) {
 #pragma unroll
         for (int e = 0; e < PER; ++e) t[e] = qr.dh.get(ks, e) * p;
         hsh[ks][lane] = M::pack(t, 0);
+      } else if constexpr (kDhRegs) {
+        hreg[ks] = qr.dh.f[ks];
       } else {
         hsh[ks][lane] = qr.dh.f[ks];
       }
@@ -331,7 +346,7 @@ void dq_kernel(BwdKArgs a) {
     // register r -> key k0 + rowof(r, half), lane -> query i
     f32x16 s, slo, dp;  // fp32: s + slo
     float ikl, iv;  // 1/|k|, 1/|v| of this lane's key row m
-    frag ka[NDH * NC];
+    frag ka[kLateK<T, DP> ? 1 : NDH * NC];
     {
       float s2k, s2v;
       {
@@ -349,7 +364,7 @@ void dq_kernel(BwdKArgs a) {
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) vf[ks] = U::row_frag(vt, rb, ks);
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) hf[ks] = hsh[ks][lane];
+        for (int ks = 0; ks < NKS; ++ks) hf[ks] = kDhRegs ? hreg[kDhRegs ? ks : 0] : hsh[kDhRegs ? 0 : ks][lane];
         zero_tail(vf);
         dp = unit_product<T>(vf, hf);
         s2v = row_dot<T>(vf, vf);
@@ -357,15 +372,16 @@ void dq_kernel(BwdKArgs a) {
         guard_keep(hf);
       }
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!kLateK<T, DP>)
 #pragma unroll
-      for (int dblk = 0; dblk < NDH; ++dblk)
+        for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) ka[dblk * NC + c] = U::col_frag(kt, cb, dblk, c);
+          for (int c = 0; c < NC; ++c) ka[dblk * NC + c] = U::col_frag(kt, cb, dblk, c);
       ikl = k0 + m < a.Tk && kmask == 0u ? inv_len_of<T>(half_sum(s2k), a.eps) : 0.0f;
       iv = inv_len_of<T>(half_sum(s2v), a.eps);
     }
-    // every read of the staged rows has returned: the next unit's copies run
-    // behind the rest of this unit's work
+    // every read of the staged rows has returned (kLateK: of the V rows): the
+    // next unit's copies run behind the rest of this unit's work
     int nxt = -1;  // this wave's next unit: S positions on in the row's walk
     for (int w = 0; w < S; ++w) {
       nxt = walk.next();
@@ -373,7 +389,7 @@ void dq_kernel(BwdKArgs a) {
     }
     wave_lds_sync();
     if (nxt >= 0) {
-      ksrc.issue(kt_at, nxt);
+      if constexpr (!kLateK<T, DP>) ksrc.issue(kt_at, nxt);
       vsrc.issue(vt_at, nxt);
       kmask = key_mask(nxt);
     }
@@ -467,12 +483,27 @@ void dq_kernel(BwdKArgs a) {
     frag db[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) db[c] = M::pack(dp, c * PER);
+    if constexpr (kLateK<T, DP>) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
+      for (int dblk = 0; dblk < NDH; ++dblk) {
+        frag f[NC];
 #pragma unroll
-      for (int dblk = 0; dblk < NDH; ++dblk) adq[dblk] = M::mma_ng(ka[dblk * NC + c], db[c], adq[dblk]);
-    guard_run(ka, adq[NDH - 1]);
-    guard_keep(db);
+        for (int c = 0; c < NC; ++c) f[c] = U::col_frag(kt, cb, dblk, c);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) adq[dblk] = M::mma_ng(f[c], db[c], adq[dblk]);
+        guard_run(f, adq[dblk]);
+      }
+      guard_keep(db);
+      wave_lds_sync();
+      if (nxt >= 0) ksrc.issue(kt_at, nxt);
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int dblk = 0; dblk < NDH; ++dblk) adq[dblk] = M::mma_ng(ka[dblk * NC + c], db[c], adq[dblk]);
+      guard_run(ka, adq[NDH - 1]);
+      guard_keep(db);
+    }
     cur = nxt;
   }
   dr_acc = wave_sum(dr_acc * ip) * (-2.0f / hp.r);
