@@ -64,15 +64,6 @@ __device__ inline void guard_frags(F (&f)[8]) {
   asm volatile(MSA_NOP16 : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]),
                "+v"(f[7]));
 }
-template <typename F, int N>
-__device__ inline void guard_frags(F (&f)[N]) {
-  static_assert(N % 16 == 0, "guard_frags: unsupported fragment count");
-#pragma unroll
-  for (int c = 0; c < N; c += 16)
-    asm volatile(MSA_NOP16 : "+v"(f[c]), "+v"(f[c + 1]), "+v"(f[c + 2]), "+v"(f[c + 3]), "+v"(f[c + 4]),
-                 "+v"(f[c + 5]), "+v"(f[c + 6]), "+v"(f[c + 7]), "+v"(f[c + 8]), "+v"(f[c + 9]), "+v"(f[c + 10]),
-                 "+v"(f[c + 11]), "+v"(f[c + 12]), "+v"(f[c + 13]), "+v"(f[c + 14]), "+v"(f[c + 15]));
-}
 template <typename F>
 __device__ inline void guard_frags(F (&f)[16]) {
   asm volatile(MSA_NOP16 : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]), "+v"(f[4]), "+v"(f[5]), "+v"(f[6]),
@@ -266,31 +257,21 @@ __device__ inline f32x16 unit_product(const typename Mma<T>::frag (&a)[N], const
 // second product contracting over the same rows.  With it, register r of lane
 // l holds source row  rowof(r, l/32) = 16*(r/8) + 8*(l/32) + r%8, so that the
 // PER consecutive registers a slot group feeds into one instruction cover
-// consecutive source rows (16-byte contiguous loads of the transposed operand).
+// consecutive source rows (UnitTile::col_frag reads the transposed operand's
+// slots in the same row order).
 __device__ inline int perm_row(int m) {
   const int g = m >> 3, hh = (m >> 2) & 1, t = m & 3;
   return 16 * (g >> 1) + 8 * hh + 4 * (g & 1) + t;
 }
-__device__ inline int rowof(int r, int half) { return 16 * (r >> 3) + 8 * half + (r & 7); }
 
-// Transpose by MFMA.  For 32 rows X held as A fragments x[ks] (lane l%32 ->
-// row perm_row(l%32), slots -> columns d = KS*ks + PER*(l/32) + e), the product
-// X P with a permutation matrix gives, per 32-column block dblk, a C block with
-// lane -> column d = 32*dblk + tcol(l%32) and register r -> X row
-// rowof(r, l/32).  Packed PER registers at a time, that is the A operand of a
-// second product that contracts over X's rows with a C block over the same
-// rows (register index = contraction index on both sides).  Products with 1
-// and sums with 0 are exact, so the values come through unchanged.
-// The column order tcol makes the second product's C block (rows = X's
-// columns) put, in each lane, the columns that lane holds of an operand row
-// fragment: register r of block dblk <-> fragment (ks, e) = creg_frag(dblk, r)
-// (see below), so a row-wise epilogue can combine the accumulator with the
-// operand fragments it already has, and store 16 contiguous bytes per group.
-template <typename T>
-__device__ inline int tcol(int m) {
-  if constexpr (sizeof(T) == 2) return perm_row(m);                 // 16*(m/16) + 8*((m>>2)&1) + ...
-  else return m;
-}
+// Column order of a transposed operand (UnitTile::col_frag): lane l of column
+// block dblk holds column 32*dblk + tcol(l%32), tcol = perm_row for the 2-byte
+// types and the identity for fp32.  The product's C block (rows = those
+// columns) then puts, in each lane, the columns that lane holds of an operand
+// row fragment: register r of block dblk <-> fragment slot (creg_ks, creg_e)
+// below, so a row-wise epilogue can combine the accumulator with the operand
+// fragments it already has, and store 16 contiguous bytes per group.
+//
 // Fragment slot (ks, e) that holds, in the same lane, the column that register
 // r of C block dblk covers when the block's rows are tcol-ordered columns.
 template <typename T>
@@ -493,12 +474,6 @@ __device__ inline float wave_sum(float v) {
   return v;
 }
 
-// Loads PER elements of type T from p (16-byte aligned for bf16), or zeros.
-template <typename T>
-__device__ inline typename Mma<T>::frag load_or_zero(const T* p, bool ok) {
-  return ok ? Mma<T>::load(p) : Mma<T>::zero();
-}
-
 __device__ inline float to_f(float x) { return x; }
 __device__ inline float to_f(bf16 x) { return (float)x; }
 __device__ inline float to_f(f16 x) { return (float)x; }
@@ -536,7 +511,7 @@ __device__ inline void store8(float* p, const float (&v)[8]) {
 }
 
 // Writes one row held in C-layout registers whose rows are tcol-ordered
-// columns (a product with a transpose_rows operand): value(dblk, r) -> column
+// columns (a product with column fragments): value(dblk, r) -> column
 // 32*dblk + (column of register r).  fn(dblk, r) gives the value.
 template <typename T, int NDH, typename Fn>
 __device__ inline void store_creg_row(T* row, int D, int half, Fn fn) {
@@ -849,76 +824,6 @@ struct UnitTile {
       }
       return v;
     }
-  }
-};
-
-// All of a 2-byte unit's column fragments (UnitTile::col_frag), as one block of
-// reads with its wait: the transposing builtin makes the compiler wait for
-// every copy in flight first, and in the group form the next tile's copies are.
-// `at` is the LDS address of the unit's rows plus col_base.
-template <typename T, int DP>
-__device__ inline void col_frags_now(typename Mma<T>::frag (&f)[DP / 16], uint32_t at) {
-  using U = UnitTile<T, DP>;
-  typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
-  typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4;
-  constexpr int R4 = 4 * U::ROWB, R16 = 16 * U::ROWB;
-  constexpr uint32_t kJ = (uint32_t)(U::swz(4) << 4);  // rows + 4
-  auto join = [](i32x2 a, i32x2 b) { return __builtin_bit_cast(typename Mma<T>::frag, i32x4{a[0], a[1], b[0], b[1]}); };
-  if constexpr (DP == 32) {
-    i32x2 x[4];
-    asm volatile("ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %5 offset:%6\n\t"
-                 "ds_read_b64_tr_b16 %2, %4 offset:%7\n\tds_read_b64_tr_b16 %3, %5 offset:%8\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
-                 : "v"(at), "v"(at ^ kJ), "n"(R4), "n"(R16), "n"(R16 + R4));
-    f[0] = join(x[0], x[1]);
-    f[1] = join(x[2], x[3]);
-  } else {
-#pragma unroll
-    for (int d = 0; d < DP / 32; d += 2) {  // column blocks d, d + 1: chunks 4 apart, as rows 4 apart
-      const uint32_t a0 = at ^ (uint32_t)(4 * d << 4), a1 = a0 ^ kJ;
-      static_assert(kJ == 4 << 4, "rows + 4 and the next column block swizzle alike");
-      i32x2 x[8];
-      asm volatile("ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %9 offset:%10\n\t"
-                   "ds_read_b64_tr_b16 %2, %8 offset:%11\n\tds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
-                   "ds_read_b64_tr_b16 %4, %9\n\tds_read_b64_tr_b16 %5, %8 offset:%10\n\t"
-                   "ds_read_b64_tr_b16 %6, %9 offset:%11\n\tds_read_b64_tr_b16 %7, %8 offset:%12\n\t"
-                   "s_waitcnt lgkmcnt(0)"
-                   : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
-                   : "v"(a0), "v"(a1), "n"(R4), "n"(R16), "n"(R16 + R4));
-      f[2 * d] = join(x[0], x[1]);
-      f[2 * d + 1] = join(x[2], x[3]);
-      f[2 * d + 2] = join(x[4], x[5]);
-      f[2 * d + 3] = join(x[6], x[7]);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Group form of a pass: the four waves of a 256-thread block hold four
-// adjacent units of one head (128 rows) and walk the other side's 64-row tiles
-// together.  A tile of two tensors X, Y (K, V or Q, dh) is staged once for the
-// block, wave w copying one of its four units; what depends on the other side
-// alone (1/|x|, the mask table of the block's 191 distances) is formed once by
-// the 256 threads.  Three tiles are in LDS: step n computes tile n while tile
-// n+1 has its factors formed and tile n+2 is copied, with one barrier a step.
-// ---------------------------------------------------------------------------
-constexpr int kGroup = 4;  // units (waves) of a block
-template <typename T, int DP>
-struct GroupStage {
-  using U = UnitTile<T, DP>;
-  static constexpr int TILEB = 4 * U::BYTES;  // X unit 0, X unit 1, Y unit 0, Y unit 1
-  static constexpr int NB = 3;
-  // 1/max(|x|, eps) of the staged tile's rows: two threads a row, X rows first
-  // (row t/2 of 128), every lane of the pair getting the value.
-  __device__ static inline float row_factor(const char* tile, int t, float eps) {
-    constexpr int CH = U::CPR / 2;  // 16-byte chunks per thread
-    const int row = t >> 1, r32 = row & 31;
-    const char* p = tile + (row >> 5) * U::BYTES + r32 * U::ROWB;
-    typename U::frag f[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c)
-      f[c] = *reinterpret_cast<const typename U::frag*>(p + ((((t & 1) * CH + c) ^ U::swz(r32)) << 4));
-    return inv_len_of<T>(group_sum<2>(row_dot<T>(f, f)), eps);
   }
 };
 

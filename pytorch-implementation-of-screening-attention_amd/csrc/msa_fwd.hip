@@ -302,10 +302,9 @@ size_t screen_plan_bytes(const Geometry& g) {
 }
 
 // ---------------------------------------------------------------------------
-// Screen operands.  Every input type screens on fp16 MFMA operands (long
-// windows of 2-byte inputs on int8 ones, below): K^ =
-// k/|k| rounded to fp16, and each raw query row rounded to fp16, so each vote
-// sees s up to their rounding: |s_screen - s| <= (u_k + u_q + u_k u_q)
+// Screen operands.  Heads of long windows of 2-byte inputs screen on int8 MFMA
+// operands (below), all others on fp16 ones: K^ = k/|k| rounded to fp16, and
+// each raw query row rounded to fp16, so each vote sees s up to their rounding: |s_screen - s| <= (u_k + u_q + u_k u_q)
 // sum_d |q^_d k^_d| <= u_k + u_q + u_k u_q (unit roundoffs, unit vectors).
 // The live-unit bitmap must hold every pair with alpha > 0 (the live and
 // backward passes visit nothing else, and a missed pair's gradient terms are
@@ -1353,8 +1352,7 @@ static hipError_t launch_fwd_t(const FwdCall& c) {
       e = screen(std::false_type{});
     if (e != hipSuccess) return e;
   }
-  // A launch with few rows (under about two waves per SIMD) splits each
-  // row's live units over S waves (DP <= 64: the S waves' LDS fits)
+  // A launch with few rows splits each row's live units over S waves
   const int64_t rows = (int64_t)2 * g.nqt * g.B * g.H;
   const int S = split_waves<T>(rows);
   const dim3 grid((unsigned)(2 * g.nqt), (unsigned)(g.B * g.H));

@@ -105,8 +105,17 @@ int decode_max_chunks(int max_len);
 hipError_t launch_decode(const DecodeCall& c);
 
 // Waves that share a row (32-query or 32-key unit) in the live, dq and dK/dV
-// passes: launches with few rows split each row's units, up to about two
-// waves per SIMD of the chip (2-byte types) or four (fp32).
+// passes: launches with few rows split each row's units, so that about 2048
+// waves (2-byte types) or 4096 (fp32, whose rows take several times as long)
+// are in flight.  us of the three passes with 1 / 2 / 4 waves, about 5% of the
+// pairs live, T = 512 and T = 1280 .. 2048 (a wave's fixed part weighs more in
+// short rows, so the best split lies lower there):
+//                 512 rows                 1024                     2048
+//   bf16 D=64     72/52/43    229/141/93   80/62/71    240/152/121  90/95/127   258/191/221
+//   bf16 D=128    102/76/86   334/207/163  114/113/161 356/242/284  164/204/311 394/414/538
+//   fp32 D=64     246/154/135 912/510/319  258/210/257 941/559/548  337/381/480 1017/943/1067
+//   fp32 D=128    508/307/292 1854/987/616 591/455/558 2054/1121/1122  829/864/1084 2395/2107/2232
+// (3072 rows of fp32: D=64 487/555/716 and 1356/1397/1575.)
 template <typename T>
 inline int split_waves(int64_t rows) {
   const int64_t most = sizeof(T) == 2 ? 2048 : 4096;
