@@ -714,9 +714,9 @@ __device__ inline void rederive(uint32_t& x) { asm volatile("" : "+v"(x)); }
 // plain 4-byte reads (fp32).  Loaded straight into operand registers instead,
 // every load instruction touches 32 rows (of fp32 4 bytes each), the next
 // unit's rows occupy registers, and each transpose costs identity MFMAs and
-// repacking.  Measured, live / dq / dK/dV: B=4, T=8192, H=8, D=64 bf16 with
-// every unit live 716 / 712 / 702 -> 504 / 693 / 478 us; B=2, T=1500 fp32
-// 207 / 370 / 440 -> 97 / 125 / 137 us.
+// repacking.  Measured, live / dq / dK/dV, before the staging and now: B=4,
+// T=8192, H=8, D=64 bf16 with every unit live 716 / 713 / 699 -> 494 / 666 / 479
+// us; B=2, T=1500 fp32 206 / 371 / 438 -> 69 / 118 / 132 us.
 // Chunks of 16 bytes are XOR-swizzled within their row (lds_swz): the DMA
 // writes linearly, so each lane fetches the chunk that belongs at its place.
 // lds_swz is linear over the row's bits, so offsets of other rows, steps and

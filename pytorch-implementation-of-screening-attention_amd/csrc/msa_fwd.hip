@@ -339,8 +339,9 @@ size_t screen_plan_bytes(const Geometry& g) {
 //     rows e_q + e_k is about 0.014, which marks about 1.6 times the units that
 //     hold a live pair; the live pass takes the others' bits back.  A bound by
 //     lengths is loose for single pairs, but the only one that never misses.
-//     B=1 T=100,000 bf16 at initialisation, windows 512 .. 100,000: screen
-//     2620 -> 1681 us, live pass 425 -> 706 (its DMA of the dead units' rows).
+//     B=1 T=100,000 bf16 at initialisation, windows 512 .. 100,000 (the narrowest
+//     head on fp16), against fp16 for all and the live pass of that time: screen
+//     2548 -> 1526 us, live pass 506 -> 701 (its DMA of the dead units' rows).
 constexpr float kKhatScale = 1024.0f;  // fp16 K^ is stored times 2^10
 constexpr float kInt8Slack = 2e-5f;    // fp32 rounding of s, |q|, |k|, e_q and e_k
 template <typename T>
@@ -396,14 +397,10 @@ __device__ inline uint32_t pack4(uint32_t a, uint32_t b, uint32_t c, uint32_t d)
 // Heads that screen on int8 operands, where the launch takes them
 // (screens_int8): windows of at least 4096 positions.  Shorter ones don't pay
 // for the heavier row preparation and the live pass's walk over units that
-// turn out dead: us a call, fp16 -> int8 for all heads: causal bf16 step at
-// initialisation, windows T/16 .. T, T = 4096 186 -> 189, T = 8192 208 -> 195
-// (D = 128: 315 -> 261); forward T = 30000 322 -> 262, with windows of
-// 32 .. 512 49 -> 57.
+// turn out dead: forward at T = 30000 with int8 for all heads, windows of
+// 32 .. 512: 49 -> 57 us.
 constexpr int kInt8Window = 4096;
-__device__ inline bool int8_window(float w, int Tq, int Tk) {
-  return w >= (float)kInt8Window && (Tq > Tk ? Tq : Tk) >= kInt8Window;
-}
+__device__ inline bool int8_window(float w) { return w >= (float)kInt8Window; }
 
 // Scale and error of a key unit's int8 rows.
 struct KeyUnitScale { float g, e; };  // g_k, e_k
@@ -423,7 +420,7 @@ __global__ __launch_bounds__(256) void prep_k_kernel(PrepKArgs a) {
   const int bh = blockIdx.y - 1, b = bh / a.H, h = bh % a.H;
   const int d0 = (threadIdx.x % CPR) * VEC;
   char* const khat = (char*)a.khat + (int64_t)bh * a.Tk_pad * DP * (int)sizeof(f16);  // the head's rows
-  const bool int8 = I8 && int8_window(a.w[h], a.Tq, a.Tk);
+  const bool int8 = I8 && int8_window(a.w[h]);
   float x[kPrepRows][VEC];
 #pragma unroll
   for (int u = 0; u < kPrepRows; ++u) {
@@ -632,7 +629,7 @@ void fwd_screen_kernel(FwdKArgs a) {
   using G = ScreenTile<S, DP>;
   constexpr int KS = M::KS, PER = M::PER, NKS = DP / KS, NS = G::NS;
   uint32_t tid_opaque = threadIdx.x;
-  if constexpr (ANY8) rederive(tid_opaque);  // one operand type's offsets don't hold registers in the other's loops
+  if constexpr (I8) rederive(tid_opaque);  // the other type's loops need their registers
   const int tid = (int)tid_opaque, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
   const int b = bh / a.H, h = bh % a.H;
   const bool causal = a.causal != 0;
@@ -958,7 +955,7 @@ void fwd_screen_kernel(FwdKArgs a) {
   guard_frags(qf);
   };
   if constexpr (ANY8) {
-    if (int8_window(head_w, a.Tq, a.Tk)) run(int8_t());
+    if (int8_window(head_w)) run(int8_t());
     else run(f16());
   } else {
     run(f16());
@@ -1079,6 +1076,7 @@ void fwd_live_kernel(FwdKArgs a) {
   }
   const float iq = qr.inv_norm(a.eps);
   const float thq = hp.thr / iq;  // s > thr  <=>  (k . q)/|k| > thr |q|
+  const bool refine = REFINE && int8_window(head_w);  // (fp16 heads mark few dead units)
   f32x16 o[NDH];
 #pragma unroll
   for (int dblk = 0; dblk < NDH; ++dblk)
@@ -1187,7 +1185,7 @@ void fwd_live_kernel(FwdKArgs a) {
       // row when S = 1, and it holds the row's words already).  A unit stays if
       // some in-window pair passes the conservative gate: a pair that is live by
       // less than the rounding of s keeps its unit marked.
-      if constexpr (REFINE) {
+      if (REFINE && refine) {
         float smax = s[0];
 #pragma unroll
         for (int r = 1; r < 16; ++r) smax = fmaxf(smax, s[r]);
@@ -1295,13 +1293,20 @@ size_t fwd_ws_bytes(const Geometry& g) { return khat_bytes(g) + screen_plan_byte
 
 // Whether heads of long windows screen on int8 operands (DP >= 64): 2-byte
 // inputs (an fp32 live pass spends more on a dead unit than the screen saves:
-// causal step T = 8192, B = 2: 277 -> 288 us), positions enough for a long
-// window, and a live pass of one wave a row without dropout, which takes the
-// dead units' bits back.
-template <typename T>
+// causal step T = 8192, B = 2: 277 -> 288 us), positions enough for long
+// windows, and a live pass of one wave a row without dropout, which takes the
+// dead units' bits back.  us of the forward's three kernels, fp16 -> int8,
+// causal bf16, H = 8, windows T/16 .. T:
+//   D = 64   B=4 T=4096 61.5 -> 70.1, T=5500 78.1 -> 83.0, T=6144 84.5 -> 82.6 (B=2
+//            63.3 -> 66.3), T=7000 107.2 -> 104.1, T=8192 123.7 -> 112.5
+//   D = 128  B=4 T=4096 81.2 -> 84.1, T=5500 118.7 -> 113.5, T=8192 212 -> 175; windows
+//            4096 .. 5000, B=8 T=5000 251 -> 192
+template <int DP>
+constexpr int kInt8Length = DP == 64 ? 7000 : kInt8Window;
+template <typename T, int DP>
 static bool screens_int8(const FwdCall& c) {
   const Geometry& g = c.g;
-  return sizeof(T) == 2 && !c.drop.on && (g.Tq > g.Tk ? g.Tq : g.Tk) >= kInt8Window &&
+  return sizeof(T) == 2 && !c.drop.on && (g.Tq > g.Tk ? g.Tq : g.Tk) >= kInt8Length<DP> &&
          split_waves<T>((int64_t)2 * g.nqt * g.B * g.H) == 1;
 }
 
@@ -1314,7 +1319,7 @@ static hipError_t launch_fwd_t(const FwdCall& c) {
   FwdKArgs fa;
   fa.q = c.q; fa.qs = c.qs; fa.k = c.k; fa.ks = c.ks; fa.v = c.v; fa.vs = c.vs; fa.kpm = c.kpm;
   fa.khat = c.khat;
-  const bool int8 = DP >= 64 && screens_int8<T>(c);
+  const bool int8 = DP >= 64 && screens_int8<T, DP>(c);
   fa.r = c.r; fa.w = c.w; fa.y = c.y; fa.hnorm = c.hnorm; fa.bits = c.bits;
   fa.H = g.H; fa.Tq = g.Tq; fa.Tk = g.Tk; fa.D = g.D; fa.nqt = g.nqt; fa.nku_words = g.nku_words;
   fa.causal = g.causal; fa.Tk_pad = g.Tk_pad; fa.eps = c.eps; fa.drop = c.drop;

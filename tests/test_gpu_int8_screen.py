@@ -1,5 +1,6 @@
 """The int8 screen (2-byte inputs, heads whose window is at least 4096
-positions, launches of one wave a row) against the float64 live-pair oracle.
+positions, launches of one wave a row over at least 7000 positions at D = 64,
+4096 at D = 128) against the float64 live-pair oracle.
 
 Every unit with a live pair must be marked; the live pass takes back the bits
 of units without one, so in int8 heads a marked unit holds a pair with
@@ -36,10 +37,10 @@ def _units(bits, B, H, Tq, Tk):
 
 
 @pytest.mark.parametrize("dtype,D,Tq,Tk,causal,padded", [
-    (torch.bfloat16, 64, 4131, 4131, True, False),
-    (torch.float16, 64, 4131, 4131, True, True),
-    (torch.bfloat16, 64, 4224, 2100, False, True),
-    (torch.float16, 64, 4200, 4200, False, False),
+    (torch.bfloat16, 64, 7013, 7013, True, False),
+    (torch.float16, 64, 7013, 7013, True, True),
+    (torch.bfloat16, 64, 7040, 2100, False, True),
+    (torch.float16, 64, 7000, 7000, False, False),
     (torch.bfloat16, 128, 4131, 4131, True, True),
     (torch.float16, 128, 4100, 4500, False, False),
 ])
@@ -104,13 +105,14 @@ def test_int8_screen_marks_the_live_units(dtype, D, Tq, Tk, causal, padded):
         assert e <= tol, f"{name}: per-head error {e:.3e} > {tol}"
 
 
+@pytest.mark.parametrize("D,T", [(64, 7040), (128, 4096)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-def test_pairs_at_the_threshold_keep_their_unit(dtype):
+def test_pairs_at_the_threshold_keep_their_unit(dtype, D, T):
     """Each head's r is the largest fp32 value at which its most similar pair is
     live in float64 (a = 1 - r(1 - s) below 2e-7): the fp32 a of such a pair is
     as often 0 as not, and its unit stays marked either way."""
     from multiscreen import ops
-    T, H, D = 4096, 16, 64
+    H = 16
     for seed in range(3):
         g = torch.Generator(device=DEV).manual_seed(seed)
         q, k, v = (torch.randn(1, T, H, D, device=DEV, generator=g).to(dtype) for _ in range(3))
