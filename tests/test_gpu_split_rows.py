@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import screening_oracle as O
-from helpers import correlated_qkv, np64, rel_err, rw64
+from helpers import correlated_qkv, errors, head_sum_err, np64, rel_err, rw64
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +38,35 @@ def test_split_rows_d128(dtype, B, drop):
     for name, got, want in zip(("y", "dq", "dk", "dv", "dr", "dw"), (y, *grads), ref):
         e = rel_err(np64(got), want)
         assert e <= TOL[dtype], f"{name}: rel err {e:.3e} > {TOL[dtype]}"
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 128), (torch.float32, 64), (torch.bfloat16, 64), (torch.float16, 32)])
+def test_rows_of_few_units(dtype, D):
+    """Rows and columns with 0, 1, 2, 3, 4 and more live units under a split over
+    four waves: those of one unit are wave 0's alone, others add up as many parts as
+    have units.  Query unit u repeats the keys of u mod 7 key units, all else is far
+    below the threshold."""
+    from multiscreen import ops
+    B, T, H, r, w = 2, 320, 2, [6.0, 7.0], [1e4, 1e5]
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(B, T, H, D, generator=g) for _ in range(3))
+    for u in range(10):
+        for n in range(min(u, u % 7)):  # key unit n, earlier than the query unit
+            q[:, 32 * u + n] = k[:, 32 * n + u] + 0.3 * torch.randn(B, H, D, generator=g)
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    dy = torch.randn(B, T, H, D, generator=g).to(dtype)
+    rg, wg = torch.tensor(r, device=DEV), torch.tensor(w, device=DEV)
+    args = [x.to(DEV) for x in (q, k, v)]
+    y, hnorm, bits = ops.fwd_raw(*args, rg, wg, True, 1e-8, None)
+    grads = ops.bwd_raw(*args, rg, wg, True, 1e-8, y, hnorm, bits, dy.to(DEV))
+    ref_args = (np64(q), np64(k), np64(v), rw64(r), rw64(w))
+    near = O.live_pairs(*ref_args[:2], *ref_args[3:], True)
+    counts = {len(set(near["j"][(near["i"] // 32 == u) & (near["b"] == 0) & (near["h"] == 0)] // 32)) for u in range(10)}
+    assert {0, 1, 2, 3, 4, 5} <= counts, counts
+    _, ref, P = O.sparse_forward_backward(*ref_args, np64(dy), True)
+    for name, got, want in zip(("dq", "dk", "dv"), grads, ref):
+        e = errors(np64(got), want)
+        assert e["max"] <= TOL[dtype] and e["fro"] <= TOL[dtype], f"{name}: {e}"
+    for name, got, want, scale in (("dr", grads[3], ref[3], P["dr_abs"]), ("dw", grads[4], ref[4], P["dw_abs"])):
+        e = head_sum_err(np64(got), want, scale)
+        assert e <= TOL[dtype], f"{name}: per-head error {e:.3e}"
