@@ -980,7 +980,7 @@ void fwd_screen_kernel(FwdKArgs a) {
 // bitwise) and runs the epilogue.
 // ---------------------------------------------------------------------------
 // REFINE (after an int8 screen; S = 1, no dropout): a unit whose pairs all lie
-// below the threshold, beyond the rounding of s, stops before its pair weights
+// below the threshold, beyond the rounding of s, stops before its value product
 // and loses its bit.
 template <typename T, int DP, int S, bool DROP, bool REFINE = false>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(unit_waves<T, DP>())))
@@ -1184,25 +1184,20 @@ void fwd_live_kernel(FwdKArgs a) {
       // reaches y or a gradient, and their bit is taken back (one wave walks a
       // row when S = 1, and it holds the row's words already).  A unit stays if
       // some in-window pair passes the conservative gate: a pair that is live by
-      // less than the rounding of s keeps its unit marked.
-      if (REFINE && refine) {
-        float smax = s[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) smax = fmaxf(smax, s[r]);
-        bool keep = __ballot(smax > thq) != 0ull;
+      // less than the rounding of s keeps its unit marked.  The vote is taken
+      // behind the weights: ahead of them it stood on the unit's dependent chain
+      // (B=1 T=18908 bf16, 5% of the pairs live: 777 us, here 736).
+      float smax = s[0];
+      if constexpr (REFINE) {
         const int c = qu * kUnit - k0;
-        if (keep && !(in_window(c - 31, hp) && in_window(c + 31, hp))) {  // a window edge cuts the unit
+        if (in_window(c - 31, hp) && in_window(c + 31, hp)) {
+#pragma unroll
+          for (int r = 1; r < 16; ++r) smax = fmaxf(smax, s[r]);
+        } else {  // a window edge cuts the unit
           smax = -INFINITY;
 #pragma unroll
           for (int r = 0; r < 16; ++r)
             smax = mrow[23 - (16 * (r >> 3) + (r & 7))] > 0.0f ? fmaxf(smax, s[r]) : smax;
-          keep = __ballot(smax > thq) != 0ull;
-        }
-        if (!keep) {
-          if (lane == 0)
-            atomicAnd(a.bits + ((int64_t)bh * 2 * a.nqt + qu) * a.nku_words + (cur >> 5), ~(1u << (cur & 31)));
-          cur = nxt;
-          continue;
         }
       }
       auto body = [&](int r) {
@@ -1221,6 +1216,14 @@ void fwd_live_kernel(FwdKArgs a) {
       } else {
 #pragma unroll
         for (int r = 0; r < 16; ++r) body(r);
+      }
+      if constexpr (REFINE) {
+        if (refine && __ballot(smax > thq) == 0ull) {
+          if (lane == 0)
+            atomicAnd(a.bits + ((int64_t)bh * 2 * a.nqt + qu) * a.nku_words + (cur >> 5), ~(1u << (cur & 31)));
+          cur = nxt;
+          continue;
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
       float vsc[16];
