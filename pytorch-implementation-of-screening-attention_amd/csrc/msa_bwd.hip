@@ -189,15 +189,6 @@ constexpr int dq_waves() { return sizeof(T) * DP <= 64 ? 3 : (sizeof(T) * DP <= 
 template <typename T, int DP>
 constexpr bool kLateK = sizeof(T) * DP > 256;
 
-// S > 1: how many of the S waves have a unit, from a copy of the walk after its
-// first unit (block-uniform: the waves walk the same bits).
-template <int S, typename Walk>
-__device__ inline int waves_with_units(Walk rest) {
-  int n = 1;
-  while (n < S && rest.next() >= 0) ++n;
-  return n;
-}
-
 template <typename T, int DP, int S, bool DROP>
 __global__ __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(dq_waves<T, DP>())))
 void dq_kernel(BwdKArgs a) {
@@ -267,9 +258,11 @@ void dq_kernel(BwdKArgs a) {
   }
   // a row of one unit, the usual one at initialisation, is wave 0's alone: the
   // others leave, and there is nothing to add up (B=8 T=241 x 269 D=64 bf16, us:
-  // one wave a row 10.2, four 14.9, four with the others gone 9.2)
-  const int nw = waves_with_units<S>(walk);
-  if (nw == 1 && wave != 0) return;
+  // one wave a row 9.2, four 14.9, four with the others gone 10.2; B=2 T=298 7.6,
+  // 9.7, 7.8).  Not for fp32, whose rows of one unit gained from the split as it is,
+  // and where the branch cost dense rows 3% (B=2 T=1500 D=64 117 -> 120).
+  const bool alone = S > 1 && sizeof(T) == 2 && walk.ended();
+  if (alone && wave != 0) return;
   for (int w = 0; w < wave && cur >= 0; ++w) cur = walk.next();  // S > 1: the wave's first unit
 
   // key row of this lane in unit u: 32u + perm_row(l32)
@@ -522,7 +515,7 @@ void dq_kernel(BwdKArgs a) {
   }
   dr_acc = wave_sum(dr_acc * ip) * (-2.0f / hp.r);
   dw_acc = wave_sum(dw_acc * ip);
-  if (S > 1 && nw > 1) {
+  if (S > 1 && !alone) {
     auto part = [&](int w) { return reinterpret_cast<float(*)[kWave]>(stage[w]); };
     if (wave > 0) {
 #pragma unroll
@@ -533,7 +526,7 @@ void dq_kernel(BwdKArgs a) {
     }
     __syncthreads();
     if (wave > 0) return;
-    for (int w = 1; w < nw; ++w) {
+    for (int w = 1; w < S; ++w) {
 #pragma unroll
       for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll
@@ -657,8 +650,8 @@ void dkdv_kernel(BwdKArgs a) {
         }
     return;
   }
-  const int nw = waves_with_units<S>(walk);
-  if (nw == 1 && wave != 0) return;  // as in dq_kernel
+  const bool alone = S > 1 && sizeof(T) == 2 && walk.ended();  // as in dq_kernel
+  if (alone && wave != 0) return;
   for (int w = 0; w < wave && cur >= 0; ++w) cur = walk.next();  // S > 1: the wave's first unit
 
   // Raw q rows past Tq read row Tq-1; their 1/|q| and dh rows (workspace,
@@ -855,7 +848,7 @@ void dkdv_kernel(BwdKArgs a) {
     cur = nxt;
   }
 
-  if (S > 1 && nw > 1) {
+  if (S > 1 && !alone) {
     auto part = [&](int w) { return reinterpret_cast<float(*)[kWave]>(stage[w]); };
     auto add_up = [&](f32x16 (&acc)[NDH]) {
       if (wave > 0)
@@ -865,7 +858,7 @@ void dkdv_kernel(BwdKArgs a) {
           for (int r = 0; r < 16; ++r) part(wave)[dblk * 16 + r][lane] = acc[dblk][r];
       __syncthreads();
       if (wave == 0)
-        for (int w = 1; w < nw; ++w)
+        for (int w = 1; w < S; ++w)
 #pragma unroll
           for (int dblk = 0; dblk < NDH; ++dblk)
 #pragma unroll

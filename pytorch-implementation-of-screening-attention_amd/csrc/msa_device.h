@@ -858,6 +858,8 @@ struct RowWalk {
       fill();
     }
   }
+  // known, without a load, that no set position is left
+  __device__ inline bool ended() const { return __ballot(word != 0u) == 0ull && w0 + 64 > (hi >> 5); }
 };
 
 // Set bits of one bitmap column: rows lo..hi of bit `sh` in the words
@@ -901,6 +903,8 @@ struct ColWalk {
       fill();
     }
   }
+  // known, without a load, that no set position is left
+  __device__ inline bool ended() const { return (m0 | m1 | m2 | m3) == 0ull && end > hi; }
 };
 
 // Balanced XCD mapping for kernels with one block per (tile, head).  Blocks
